@@ -86,7 +86,10 @@ typedef struct rsh_frame_config {
     float cell_scale[3];            /* cells per world unit                              */
     uint32_t segment_shift;         /* batches: key bit of the view id (0 = not in key) */
     float initial_radius, initial_spread;
-    uint32_t traversal_kernel;      /* 0 automatic, 1 generic kernel for every shape     */
+    uint32_t traversal_kernel;      /* 0 automatic, 1 generic kernel for every shape.  The
+                                       automatic traversal walks a tree over the scene's
+                                       triangles unless one of the three fields below or
+                                       counters (flag bit 1) are asked for                */
     uint32_t traversal_splits;      /* generic kernel: waves per top node; 0 = fill the GPU */
     uint32_t traversal_chunk;       /* 64-ray kernel: candidate clusters (64 consecutive
                                        triangles of one object) per work item; 0 = sized
@@ -99,10 +102,11 @@ typedef struct rsh_frame_config {
                                        EPS, short of a shadow ray's length or the closest
                                        hit so far); 3 that and, per passing cluster,
                                        the rays' lines against the cluster's sphere (for
-                                       spread-out rays); 0 automatic: 2 for a frame's
-                                       camera rays; otherwise 3 when more than a
-                                       sixteenth of the top nodes' cones have tan(spread)
-                                       outside [0, 0.1], else 2.  Hit records
+                                       spread-out rays); 0 automatic: the triangle tree,
+                                       and where counters or a work split are asked for 2
+                                       for a frame's camera rays; otherwise 3 when more
+                                       than a sixteenth of the top nodes' cones have
+                                       tan(spread) outside [0, 0.1], else 2.  Hit records
                                        are the same in every mode; with mode 3 and stats
                                        counters (flag bit 1) the cluster masks are off so
                                        that the counts stay the reference's.             */
@@ -139,8 +143,9 @@ typedef struct rsh_frame_stats {
     uint32_t graph_replayed;                     /* 1: the call replayed a captured graph (bit 3) */
     uint64_t pass_mt_tests[RSH_MAX_PASSES];      /* Moller-Trumbore tests run after the ray pre-test
                                                     (bit 1; equals pass_ray_tests without it)   */
-    uint32_t pass_mode[RSH_MAX_PASSES];          /* 64-ray kernel mode used: 0 exact tests only,
-                                                    1 triangle pre-test, 2 and cluster masks   */
+    uint32_t pass_mode[RSH_MAX_PASSES];          /* traversal used: 3 triangle tree; 64-ray kernel:
+                                                    0 exact tests only, 1 triangle pre-test, 2 and
+                                                    cluster masks                              */
 } rsh_frame_stats;
 
 typedef struct rsh_engine rsh_engine;

@@ -131,6 +131,7 @@ struct rsh_engine {
     uint32_t T = 0, K = 0, M = 0, L = 0;
     DevBuf tri_pos, tri_nrm, tri_mat, mat_dif, mat_spec, light_pos, light_col, light_int;
     DevBuf tri_sphere, tri_mt, obj_sphere, obj_range;
+    TreeBuild tree;                    // triangle tree of the automatic traversal
     std::vector<float> host_light_pos;   // float4[L] as loaded
     // cluster level: CLUSTER consecutive triangles of one object per cluster
     uint32_t NC = 0;
@@ -793,6 +794,28 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         LANE_OK(keep(k.nodes, L.nodes.p, (size_t)2 * nn * 16));
         k.order_set = true;
     }
+    // The automatic traversal walks the triangle tree; a caller that counts
+    // the reference's tests or picks a kernel, a work split or a pre-test gets
+    // the kernels these belong to.
+    if (!counting && cfg.traversal_kernel == 0 && cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 &&
+        cfg.traversal_splits == 0) {
+        TreeParams q{};
+        q.tree = e->tree.nodes.as<TreeNode>(); q.records = f4p(e->tree.records); q.bounds = u32p(e->tree.bounds);
+        q.nodes = f4p(L.nodes); q.aux = L.aux.as<float2>();
+        for (int k = 0; k < 4; k++) q.level_offset[k] = offs[k];
+        q.depth = cfg.depth; q.branch = cfg.branch; q.rays_per_top = cfg.leaf;
+        for (uint32_t k = 1; k < cfg.depth; k++) q.rays_per_top *= cfg.branch;
+        q.rec0 = f4p(L.rec0); q.rec1 = f4p(L.rec1); q.N = N; q.T = e->T; q.ps = psz;
+        q.obj_sphere = f4p(e->obj_sphere); q.obj_range = e->obj_range.as<uint4>();
+        q.algorithm = cfg.algorithm; q.kind = kind; q.hit_mode = cfg.hit_mode;
+        q.line_only = RSH_CAMERA_LINE_ONLY && camera && kind == 0 ? 1u : 0u;
+        q.closest = u64p(closest); q.shadow = u32p(closest);       // by kind
+        StageTimer t(L, ST_PASS_TRAVERSE + (int)pass_idx, trav_timing);
+        launch_tree_trace(q, s);
+        LANE_OK(hipGetLastError());
+        out.mode = 3;
+        return RSH_OK;
+    }
     TravParams p{};
     p.nodes = f4p(L.nodes); p.aux = L.aux.as<float2>();
     for (int k = 0; k < 4; k++) { p.level_offset[k] = offs[k]; p.level_count[k] = counts[k]; }
@@ -963,6 +986,7 @@ void rsh_engine_destroy(rsh_engine* e) {
                       &e->closest[1], &e->shadow[0], &e->shadow[1], &e->pixels, &e->views_d, &e->crange, &e->srange, &e->tri_pos0,
                       &e->tri_nrm0, &e->tri_obj, &e->sph0, &e->mats, &e->sph_tmp})
         b->release();
+    e->tree.release();
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
     for (int i = 0; i < 4; i++) { e->g0[i].release(); e->gb[0][i].release(); e->gb[1][i].release(); }
@@ -1113,6 +1137,8 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     HIP_OK(hipMemcpyAsync(e->cl_base.p, base.data(), (size_t)K * 4, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(e->all_list.p, ident.data(), (size_t)K * 16, hipMemcpyHostToDevice, st));
     build_clusters(e, st);
+    HIP_OK(e->tree.reserve(T));
+    HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
     e->orig_ready = false;
@@ -1876,6 +1902,7 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
     HIP_OK(hipMemcpy2DAsync(e->obj_sphere.p, 16, e->sph_tmp.p, 24, 16, K, hipMemcpyDeviceToDevice, st));
     launch_triangle_prep(f4p(e->tri_pos), T, f4p(e->tri_sphere), f4p(e->tri_mt), st);
     build_clusters(e, st);
+    HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
     drop_graph(e);

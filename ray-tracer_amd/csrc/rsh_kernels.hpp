@@ -305,6 +305,46 @@ void launch_hits_intersect(const float* rays, const uint32_t* svalues, const uin
                            uint32_t hitTotal, uint32_t N, uint32_t offset, uint32_t W, uint32_t Lmax, uint32_t leaf,
                            const float4* gpos, uint32_t shadow, uint32_t* out, hipStream_t s);
 
+// --- triangle tree (k_tree.hip) ---
+// A four-wide node: per child (lo xyz, word), (hi xyz, -).  Word: node index,
+// or leaf flag | (triangles - 1) << 29 | first record; all ones: no child.
+struct TreeNode {
+    float4 child[4][2];
+};
+static_assert(sizeof(TreeNode) == 128, "a node is one cache line");
+
+struct TreeBuild {
+    DevBuf nodes, records, bounds;                                          // what the traversal reads (parts of keep)
+    DevBuf box, blk, codes, ids, scodes, sids, range, child, queue, count;  // construction (parts of work)
+    ScanScratch sc;                                                         // the sort's scratch (part of work)
+    DevBuf keep, work;
+    hipError_t reserve(uint32_t T);
+    // objects: per object (first triangle, ...), K of them tiling [0, T) in order
+    hipError_t build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
+                     hipStream_t s);
+    void release();
+};
+
+struct TreeParams {
+    const TreeNode* tree;
+    const float4* records;        // [4T] triangles in tree order
+    const uint32_t* bounds;
+    const float4* nodes;          // ray hierarchy, as in TravParams
+    const float2* aux;
+    uint32_t level_offset[4];
+    uint32_t depth, branch, rays_per_top;
+    const float4* rec0;
+    const float4* rec1;
+    uint32_t N, T;
+    const PassSizes* ps;          // device-sized: N and level_offset from here, N above the capacity
+    const float4* obj_sphere;
+    const uint4* obj_range;
+    uint32_t algorithm, kind, hit_mode, line_only;
+    unsigned long long* closest;  // kind 0: every traced ray's record is written
+    uint32_t* shadow;             // kind 1: MISS32 where occluded
+};
+void launch_tree_trace(const TreeParams& p, hipStream_t s);
+
 // Hierarchy level sizes: level 0 has ceil(N/leaf) nodes, level k
 // ceil(count[k-1]/branch); offsets are prefix sums.  Returns the node total.
 inline uint32_t level_sizes(uint32_t N, uint32_t leaf, uint32_t branch, uint32_t depth, uint32_t* counts,

@@ -19,7 +19,7 @@ CSRC = os.path.join(ROOT, "csrc")
 LIBDIR = os.path.join(ROOT, "lib")
 OBJDIR = os.path.join(ROOT, "lib", "obj")
 LIB = os.path.join(LIBDIR, "librsh.so")
-SOURCES = ["k_scan.hip", "k_trav.hip", "k_rays.hip", "engine.hip", "compat.hip", "server.hip", "selfcheck.hip",
+SOURCES = ["k_scan.hip", "k_trav.hip", "k_tree.hip", "k_rays.hip", "engine.hip", "compat.hip", "server.hip", "selfcheck.hip",
            "spheres.hip", "noalloc.hip"]
 ARCH = "gfx950"
 FLAGS = [

@@ -1,0 +1,161 @@
+"""The automatic traversal (triangle tree) against the kernel that tests every
+candidate (traversal_prefilter 1, itself checked against the oracle): equal
+records, bit for bit, at the sizes where the tree's construction and the
+quads' remainders can go wrong, and for rays and scenes outside the ordinary."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from rsh_amd import queries
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def engine(rsh):
+    e = rsh.Engine(0)
+    yield e
+    e.close()
+
+
+def make_scene(rsh, tris, per_object):
+    """A scene of the given [T, 3, 3] vertices, per_object consecutive triangles each."""
+    T = len(tris)
+    v = np.zeros((T, 3, 4), np.float32)
+    v[:, :, :3] = tris
+    n = np.cross(tris[:, 1] - tris[:, 0], tris[:, 2] - tris[:, 0])
+    n /= np.maximum(np.linalg.norm(n, axis=1, keepdims=True), 1e-12)
+    nrm = np.zeros((T, 3, 4), np.float32)
+    nrm[:, :, :3] = n[:, None]
+    spheres = []
+    for a in range(0, T, per_object):
+        b = min(a + per_object, T) - 1
+        p = tris[a:b + 1].reshape(-1, 3).astype(np.float64)
+        c = (p.min(0) + p.max(0)) / 2
+        spheres.append([*c, np.linalg.norm(p - c, axis=1).max() * 1.0001 + 1e-4, a, b])
+    base = rsh.scenes.config0_scene()
+    lo, hi = tris.reshape(-1, 3).min(0), tris.reshape(-1, 3).max(0)
+    return dataclasses.replace(base, tri_pos=v.reshape(-1, 4), tri_nrm=nrm.reshape(-1, 4),
+                               tri_mat=np.zeros(3 * T, np.int32), object_spheres=np.asarray(spheres, np.float32),
+                               bounds_min=lo - 1.0, bounds_max=hi + 1.0)
+
+
+def soup(rng, T, spread=100.0, size=5.0):
+    c = rng.uniform(50.0, 50.0 + spread, (T, 1, 3))
+    return (c + rng.normal(0.0, size, (T, 3, 3))).astype(np.float32)
+
+
+def rays_at(rng, sc, n):
+    o = rng.uniform(sc.bounds_min, sc.bounds_max, (n, 3))
+    t = sc.tri_pos[:, :3].reshape(-1, 3, 3).mean(1)[rng.integers(sc.triangle_total, size=n)]
+    d = t + rng.normal(0.0, 1.0, (n, 3)) - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    return np.concatenate([o, d], 1).astype(np.float32)
+
+
+def qcfg(rsh, sc, **kw):
+    return dataclasses.replace(rsh.config.config0(8, 8), cell_bits=4, dir_bits=6, **kw).with_scene_bounds(sc)
+
+
+def check(engine, rsh, sc, rays, **kw):
+    cfg = qcfg(rsh, sc, **kw)
+    engine.load_scene(sc)
+    tmax = np.full(len(rays), 60.0, np.float32)
+    for kind in (0, 1):
+        got = engine.trace(rays, kind, cfg, tmax=tmax)
+        want = engine.trace(rays, kind, dataclasses.replace(cfg, traversal_prefilter=1), tmax=tmax)
+        np.testing.assert_array_equal(got, want)
+    return want
+
+
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 8, 9, 63, 65, 513, 4099, 20011])
+def test_scene_sizes(engine, rsh, T):
+    rng = np.random.default_rng(T)
+    sc = make_scene(rsh, soup(rng, T), 7)
+    check(engine, rsh, sc, rays_at(rng, sc, 1501))
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 1025])
+def test_ray_counts(engine, rsh, n):
+    rng = np.random.default_rng(n)
+    sc = make_scene(rsh, soup(rng, 777), 50)
+    check(engine, rsh, sc, rays_at(rng, sc, n))
+
+
+@pytest.mark.parametrize("variant", [dict(algorithm=1), dict(hit_mode=1), dict(depth=1), dict(depth=3, branch=4),
+                                     dict(depth=4, leaf=4, branch=3), dict(leaf=32, branch=2), dict(key_mode=0),
+                                     dict(triangle_batch=512), dict(cone_mode=0)])
+def test_options(engine, rsh, variant):
+    rng = np.random.default_rng(3)
+    sc = make_scene(rsh, soup(rng, 3001), 64)
+    check(engine, rsh, sc, rays_at(rng, sc, 2003), **variant)
+
+
+def test_scenes_outside_the_ordinary(engine, rsh):
+    rng = np.random.default_rng(5)
+    one = soup(rng, 1)
+    flat = soup(rng, 600)
+    flat[:, :, 1] = 70.0                                     # a flat scene box
+    sliver = soup(rng, 600)
+    sliver[:, 2] = sliver[:, 1] + 1e-3                       # no reliable plane
+    point = soup(rng, 600)
+    point[::3, 1] = point[::3, 0]                            # triangles without area
+    # nested triangles about one corner, each half the size of the one before:
+    # the deepest tree the codes allow, every box on the way of the rays
+    s = 0.5 ** np.repeat(np.arange(9), 40)[:, None, None]
+    nested = (50.0 + 100.0 * s * (np.asarray([[0.1, 0.1, 0.1], [1.0, 0.1, 0.2], [0.1, 1.0, 0.3]])
+                                  + 0.01 * rng.random((360, 3, 3)))).astype(np.float32)
+    for tris in (np.repeat(one, 3000, 0), flat, sliver, point, nested):
+        sc = make_scene(rsh, tris, 30)
+        check(engine, rsh, sc, rays_at(rng, sc, 700))
+
+
+def test_rays_outside_the_ordinary(engine, rsh):
+    """Long, short, axis-parallel, zero and non-finite rays among ordinary ones."""
+    rng = np.random.default_rng(6)
+    sc = make_scene(rsh, soup(rng, 400), 40)
+    rays = rays_at(rng, sc, 640)
+    rays[0:64, 3:] *= 1e6
+    rays[64:128, 3:] *= 1e-4
+    rays[128:192, 3:] = np.eye(3, dtype=np.float32)[rng.integers(3, size=64)]
+    rays[192:256, 3:] = -np.eye(3, dtype=np.float32)[rng.integers(3, size=64)]
+    rays[256:264, 3:] = 0.0
+    rays[264:272, 3:] = np.nan
+    rays[272:280, 3] = np.inf
+    rays[280:288, 0] = np.nan
+    rays[288:296, 1] = -np.inf
+    rays[296:304, 3:] *= 1e-20
+    rays[304:312, 3:] *= 1e20
+    rays[312:320, :3] *= 1e16
+    check(engine, rsh, sc, rays)
+
+
+def test_moved_objects(engine, rsh):
+    """The tree follows the objects: a frame after an update equals the frame
+    of the exhaustive kernel on the same engine."""
+    sc = rsh.scenes.config1_scene(boxes=120)
+    cam = rsh.scenes.config1_camera(97, 61)
+    cfg = rsh.config.config1(97, 61).with_scene_bounds(sc)
+    engine.load_scene(sc)
+    K = sc.object_total
+    rng = np.random.default_rng(8)
+    for _ in range(2):
+        m = np.tile(np.eye(4, dtype=np.float32), (K, 1, 1))
+        n, s = m.copy(), m.copy()
+        m[1:, :3, 3] = rng.uniform(-20.0, 20.0, (K - 1, 3))
+        engine.update_objects(m, n, s)
+        engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+        got = [engine.pass_hits(i) for i in range(engine.stats.pass_count)]
+        engine.render(cam, dataclasses.replace(cfg, traversal_prefilter=1), flags=engine.KEEP_PASSES)
+        assert len(got) == engine.stats.pass_count
+        for i, g in enumerate(got):
+            np.testing.assert_array_equal(g, engine.pass_hits(i))
+
+
+def test_serving_mix_on_the_soup(engine, rsh):
+    """Overlapping triangles: the tree's longest paths."""
+    sc = rsh.scenes.soup_scene(triangles=30_000)
+    for mix in (queries.PRIMARY, queries.DIFFUSE):
+        rays, _, _ = queries.make_query(sc, mix, 5003, np.random.default_rng(9))
+        check(engine, rsh, sc, rays)

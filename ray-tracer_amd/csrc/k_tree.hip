@@ -346,8 +346,12 @@ __global__ void __launch_bounds__(1024) k_tree_tail(EmitArgs A, uint32_t level, 
 // triangle q of a leaf; 16 rays, one wave, per workgroup.  Nearest child first;
 // the others wait on the ray's stack in LDS.
 // Large passes are bound by VALU issue (1080p atrium camera pass: 308M
-// instructions, 0.50 ms of issue in 0.60 ms), small ones by the latency of the
-// longest ray's steps (14k rays: 0.12 ms).  One thread per ray needs half the
+// instructions, 0.50 ms of issue in 0.60 ms) and the loads behind it, small
+// ones by the latency of the longest ray's steps (14k rays: 0.12 ms).  Waves
+// hide that latency: 8 a SIMD (64 VGPRs, 9 of the closest-hit kernel's spilled;
+// 3.0 / 4.5 KB of LDS) against 7 with 6 KB: 1080p atrium frame 2.97 -> 2.92 ms,
+// 16-view batch 8.65 -> 8.08, 1M diffuse rays 0.863 -> 0.806, soft shadows 3.45 ->
+// 3.15; 6 waves 2 to 4 % slower than 7, 5 waves 6 to 10 %.  One thread per ray needs half the
 // instructions but waits twice as long per step: its seven or eight loads of a
 // node touch 64 lines each, and a leaf's triangles follow one another (same
 // camera pass 0.62-0.76 ms, the 14k rays 0.28 ms).  Against the work-item kernel
@@ -430,11 +434,18 @@ __device__ __forceinline__ bool meets(const Slabs& s, float4 lo, float4 hi, floa
 }
 
 template <int KIND>
-__global__ void __launch_bounds__(64) k_tree_trace(const TreeParams P) {
-    __shared__ uint2 s_stack[STACK][16];       // (word, entry distance)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace(const TreeParams P) {
+    __shared__ uint32_t s_stack[STACK][16];
+    __shared__ uint16_t s_near[KIND == 0 ? STACK : 1][16];     // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, ray = lane >> 2;
     const uint32_t* off = P.ps ? P.ps->offset : P.level_offset;
-    const uint32_t pos = blockIdx.x * 16 + ray;
+    // Workgroups go to the 8 XCDs in turn; 64 neighbours (1024 sorted rays) stay
+    // on one, whose L2 then holds their part of the tree (atrium frame 2.91 ->
+    // 2.86 ms; an eighth of the pass on each XCD: 2.95, and 12 % slower on the
+    // batch, whose parts differ in length).
+    const uint32_t b = blockIdx.x;
+    const uint32_t blk = b < (gridDim.x & ~511u) ? (b & ~511u) | ((b & 7u) << 6) | ((b >> 3) & 63u) : b;
+    const uint32_t pos = blk * 16 + ray;
     if (pos >= (P.ps ? P.ps->N : P.N)) return;
     const float4 r0 = P.rec0[pos], r1 = P.rec1[pos];
     const uint32_t slot = __float_as_uint(r0.w);
@@ -458,8 +469,7 @@ __global__ void __launch_bounds__(64) k_tree_trace(const TreeParams P) {
     auto pop = [&]() -> uint32_t {
         while (sp > 0) {
             sp--;
-            const uint2 w = s_stack[sp][ray];
-            if (KIND == 1 || !(__uint_as_float(w.y) > lim)) return w.x;
+            if (KIND == 1 || !(__uint_as_float((uint32_t)s_near[sp][ray] << 16) > lim)) return s_stack[sp][ray];
         }
         return TREE_EMPTY;
     };
@@ -478,12 +488,16 @@ __global__ void __launch_bounds__(64) k_tree_trace(const TreeParams P) {
             const uint32_t rank = (quad_u<QUAD_ROT1>(key) < key ? 1u : 0u) + (quad_u<QUAD_ROT2>(key) < key ? 1u : 0u) +
                                   (quad_u<QUAD_ROT3>(key) < key ? 1u : 0u);
             const bool full = sp + n > STACK;  // no ray of a scene of ordinary depth
-            if (in && !full) s_stack[sp + n - 1u - rank][ray] = make_uint2(ch, __float_as_uint(tn));
+            if (in && !full) {
+                const uint32_t at = sp + n - 1u - rank;
+                s_stack[at][ray] = ch;
+                if (KIND == 0) s_near[at][ray] = (uint16_t)(__float_as_uint(tn) >> 16);
+            }
             sp = full ? 0u : sp + n;
             n = full ? 0u : n;
             scan = full ? 0u : scan;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // pushed by one lane, popped by four
-            if (n != 0u) cur = s_stack[--sp][ray].x;
+            if (n != 0u) cur = s_stack[--sp][ray];
             else cur = pop();
         }
         if (cur == TREE_EMPTY) {
@@ -515,10 +529,10 @@ __global__ void __launch_bounds__(64) k_tree_trace(const TreeParams P) {
         const uint32_t j = first + (q < n ? q : 0u);
         const float4* rec = P.records + 4 * (size_t)j;
         const float4 sph = rec[0];
-        const float4 A = rec[1], B = rec[2], C = rec[3];
         const bool may = q < n && (P.line_only ? ray_may_hit_sphere(o, d, dd, sph)
                                                : ray_may_hit_sphere_range(o, d, dd, sph, EPS, hi));
         if (may) {
+            const float4 A = rec[1], B = rec[2], C = rec[3];
             const float th = ray_triangle(o, d, xyz(A), xyz(B), xyz(C));
             const uint32_t tri = __float_as_uint(A.w);
             unsigned long long rc = miss;

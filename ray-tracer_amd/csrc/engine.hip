@@ -673,6 +673,17 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     // unique: trimming and compression are the identity, so the slots are
     // sorted directly and no sizes are read back.
     const bool all_unique = camera && kind == 0;
+    // Device-sized pass (a capture for any camera): N and C stay in device
+    // memory; the launches below cover the pass's S slots.  The camera pass's
+    // sizes are fixed (every slot live, one chunk per ray), but its work list
+    // depends on the camera, so it takes the same path.
+    const bool dev = e->dev_sized && cfg.algorithm == RSH_CRSH && S > 0;
+    // sorted as rays or as packets (always packets where their order is read
+    // back or the sizes stay on the device)
+    PackOrder order = PACK_CHUNKS;
+    if (cfg.algorithm == RSH_CRSH && !dev && !(flags_mask & 64u))
+        order = !e->replaying ? PACK_EITHER
+                : sorts_rays(L.plan[L.plan_pos].N, L.plan[L.plan_pos].C) ? PACK_RAYS : PACK_CHUNKS;
     if (all_unique) {
         // hit records cleared: no trim or compression to time
         launch_fill_u64(u64p(closest), cfg.hit_mode == 0 ? MISS64 : (unsigned long long)MISS32, S, s);
@@ -688,13 +699,8 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         LANE_OK(run_pack(u8p(L.flags), u32p(L.keys), nullptr, S, u32p(L.tvalues), u32p(L.bases),
                         u32p(L.ckeys), u32p(L.cvalues), dc, kind == 0 ? u64p(closest) : nullptr, miss,
                         kind == 1 ? u32p(closest) : nullptr, L.sc, s, poll ? L.hsize_dev : nullptr,
-                        poll ? ++L.hseq : 0u));
+                        poll ? ++L.hseq : 0u, order));
     }
-    // Device-sized pass (a capture for any camera): N and C stay in device
-    // memory; the launches below cover the pass's S slots.  The camera pass's
-    // sizes are fixed (every slot live, one chunk per ray), but its work list
-    // depends on the camera, so it takes the same path.
-    const bool dev = e->dev_sized && cfg.algorithm == RSH_CRSH && S > 0;
     PassSizes* psz = dev ? L.psz.as<PassSizes>() : nullptr;
     if (dev && all_unique)
         launch_fixed_sizes(S, S, cfg.leaf, cfg.branch, cfg.depth, psz, u32p(e->frame_rec) + 2 * (size_t)pass_idx, s);
@@ -728,6 +734,12 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         out.C = N;
         StageTimer t(L, ST_SORT, timing);
         LANE_OK(run_radix_sort(u32p(L.keys), u32p(L.values), N, sort_bits ? sort_bits : key_bits(cfg), u32p(L.skeys),
+                               u32p(L.svalues), L.sc, s));
+        sorted_values = u32p(L.svalues);
+    } else if (order == PACK_RAYS || (order == PACK_EITHER && sorts_rays(N, hc[1]))) {
+        out.C = hc[1];
+        StageTimer t(L, ST_SORT, timing);
+        LANE_OK(run_radix_sort(u32p(L.ckeys), u32p(L.cvalues), N, sort_bits ? sort_bits : key_bits(cfg), u32p(L.skeys),
                                u32p(L.svalues), L.sc, s));
         sorted_values = u32p(L.svalues);
     } else if (cfg.algorithm == RSH_CRSH) {

@@ -514,7 +514,8 @@ __global__ void __launch_bounds__(256) k_pack_write(const uint8_t* flags, const 
                                                     const uint32_t* values, uint64_t n, const uint4* meta,
                                                     uint32_t* tvalues, uint32_t* bases, uint32_t* ckeys,
                                                     uint32_t* cvalues, unsigned long long* clear64,
-                                                    unsigned long long miss, uint32_t* clear32) {
+                                                    unsigned long long miss, uint32_t* clear32, uint32_t order,
+                                                    const uint32_t* totals) {
     __shared__ uint32_t sa[TILE];
     __shared__ uint32_t sb[TILE];
     __shared__ LastKey lk[WAVES];
@@ -559,6 +560,18 @@ __global__ void __launch_bounds__(256) k_pack_write(const uint8_t* flags, const 
     const uint32_t ex = block_excl_sum((nh << 16) | nl, red, &total);
     const uint32_t tl = total & 0xFFFFu, th = total >> 16;
     uint32_t lp = ex & 0xFFFFu;
+    // one (key, value) pair per live ray: they are sorted directly
+    if (order == PACK_RAYS || (order == PACK_EITHER && sorts_rays(totals[0], totals[1]))) {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (t.live & (1u << i)) { sa[lp] = v[i]; sb[lp++] = k[i]; }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < tl; i += blockDim.x) {
+            ckeys[m.x + i] = sb[i];
+            cvalues[m.x + i] = sa[i];
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 16; i++)
         if (t.live & (1u << i)) sa[lp++] = v[i];
@@ -709,10 +722,10 @@ __global__ void __launch_bounds__(256) k_unpack_expand(const uint32_t* soff, con
 // key in three passes instead of four); DPT = digits per thread of a
 // 256-thread block in the per-digit steps, each thread owning DPT
 // consecutive digits so that a block scan keeps digit order.
-template <uint32_t RB>
+template <uint32_t RB, uint32_t ITEMS>
 __global__ void __launch_bounds__(256) k_radix_upsweep(const uint32_t* keys, uint64_t n, uint32_t shift,
                                                        uint32_t* hist, uint32_t ntiles, const uint32_t* d_n) {
-    constexpr uint32_t NB = 1u << RB, MASK = NB - 1u;
+    constexpr uint32_t NB = 1u << RB, MASK = NB - 1u, TS = 256u * ITEMS;
     if (d_n) {                            // device-sized: n and the tile count from memory
         n = min(n, (uint64_t)*d_n);
         ntiles = tiles_of((uint32_t)n);
@@ -722,15 +735,15 @@ __global__ void __launch_bounds__(256) k_radix_upsweep(const uint32_t* keys, uin
     for (uint32_t i = threadIdx.x; i < WAVES * NB; i += blockDim.x) (&cnt[0][0])[i] = 0;
     __syncthreads();
     const uint32_t w = wave_id(), lane = lane_id();
-    const uint64_t tb = (uint64_t)blockIdx.x * TILE + (uint64_t)w * 1024;
-    uint32_t k[16];      // all loads issued before the first use
+    const uint64_t tb = (uint64_t)blockIdx.x * TS + (uint64_t)w * (64u * ITEMS);
+    uint32_t k[ITEMS];   // all loads issued before the first use
 #pragma unroll
-    for (uint32_t r = 0; r < 16; r++) {
+    for (uint32_t r = 0; r < ITEMS; r++) {
         const uint64_t p = tb + r * 64 + lane;
         k[r] = p < n ? keys[p] : 0u;
     }
 #pragma unroll
-    for (uint32_t r = 0; r < 16; r++)
+    for (uint32_t r = 0; r < ITEMS; r++)
         if (tb + r * 64 + lane < n) atomicAdd(&cnt[w][(k[r] >> shift) & MASK], 1u);
     __syncthreads();
     for (uint32_t d = threadIdx.x; d < NB; d += blockDim.x) {
@@ -761,12 +774,12 @@ __global__ void __launch_bounds__(256) k_radix_rowscan(uint32_t* hist, uint32_t 
 
 // ROWSCAN: hist holds the upsweep's raw tile counts and each block sums its
 // digit rows itself (for small tile counts, in place of k_radix_rowscan).
-template <bool ROWSCAN, uint32_t RB>
+template <bool ROWSCAN, uint32_t RB, uint32_t ITEMS>
 __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, const uint32_t* vals, uint64_t n,
                                                          uint32_t shift, const uint32_t* hist, uint32_t ntiles,
                                                          const uint32_t* digit_totals, uint32_t* okeys,
                                                          uint32_t* ovals, const uint32_t* d_n) {
-    constexpr uint32_t NB = 1u << RB, MASK = NB - 1u, DPT = NB / 256u;
+    constexpr uint32_t NB = 1u << RB, MASK = NB - 1u, DPT = NB / 256u, TS = 256u * ITEMS;
     if (d_n) {
         n = min(n, (uint64_t)*d_n);
         ntiles = tiles_of((uint32_t)n);
@@ -775,8 +788,8 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
     __shared__ uint32_t whist[WAVES][NB];
     __shared__ uint32_t tile_start[NB];
     __shared__ uint32_t gbase[NB];
-    __shared__ uint32_t sk[TILE];
-    __shared__ uint32_t sv[TILE];
+    __shared__ uint32_t sk[TS];
+    __shared__ uint32_t sv[TS];
     __shared__ uint32_t lds[WAVES];
     const uint32_t tid = threadIdx.x, w = wave_id(), lane = lane_id();
     for (uint32_t i = tid; i < WAVES * NB; i += blockDim.x) (&whist[0][0])[i] = 0;
@@ -810,17 +823,17 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
         }
     }
     __syncthreads();
-    const uint64_t tb = (uint64_t)blockIdx.x * TILE + (uint64_t)w * 1024;
+    const uint64_t tb = (uint64_t)blockIdx.x * TS + (uint64_t)w * (64u * ITEMS);
     const uint64_t lt = (1ull << lane) - 1ull;
-    uint32_t key[16], val[16], rank[16];
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
 #pragma unroll
-    for (uint32_t r = 0; r < 16; r++) {      // all loads issued before the ranking
+    for (uint32_t r = 0; r < ITEMS; r++) {      // all loads issued before the ranking
         const uint64_t p = tb + r * 64 + lane;
         key[r] = p < n ? keys[p] : 0u;
         val[r] = p < n ? vals[p] : 0u;
     }
 #pragma unroll
-    for (uint32_t r = 0; r < 16; r++) {
+    for (uint32_t r = 0; r < ITEMS; r++) {
         uint64_t p = tb + r * 64 + lane;
         bool valid = p < n;
         uint32_t k = key[r];
@@ -861,7 +874,7 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
     }
     __syncthreads();
 #pragma unroll
-    for (uint32_t r = 0; r < 16; r++) {
+    for (uint32_t r = 0; r < ITEMS; r++) {
         uint64_t p = tb + r * 64 + lane;
         if (p < n) {
             uint32_t d = (key[r] >> shift) & MASK;
@@ -871,8 +884,8 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
         }
     }
     __syncthreads();
-    const uint64_t tile0 = (uint64_t)blockIdx.x * TILE;
-    const uint32_t valid_n = (uint32_t)((n - tile0) < TILE ? (n - tile0) : TILE);
+    const uint64_t tile0 = (uint64_t)blockIdx.x * TS;
+    const uint32_t valid_n = (uint32_t)((n - tile0) < TS ? (n - tile0) : TS);
     for (uint32_t i = tid; i < valid_n; i += blockDim.x) {
         uint32_t k = sk[i];
         uint32_t d = (k >> shift) & MASK;
@@ -935,8 +948,7 @@ inline uint32_t grid_for(uint64_t n, uint32_t block, uint32_t cap = 1u << 20) {
 hipError_t ScanScratch::reserve(uint64_t n) {
     hipError_t e;
     if ((e = tile_counts.reserve((MAX_TILES + 1) * sizeof(uint32_t))) != hipSuccess) return e;
-    uint32_t nt = tiles_for(n) + 1;
-    if ((e = hist.reserve((size_t)512 * nt * sizeof(uint32_t))) != hipSuccess) return e;    // 9-bit digits
+    if ((e = hist.reserve(sort_hist_bytes(n))) != hipSuccess) return e;
     if ((e = digit_totals.reserve(512 * sizeof(uint32_t))) != hipSuccess) return e;
     if ((e = total.reserve(4 * sizeof(uint32_t))) != hipSuccess) return e;
     if ((e = ping_k.reserve(n * sizeof(uint32_t))) != hipSuccess) return e;
@@ -1035,7 +1047,7 @@ hipError_t run_compress(const uint32_t* keys, uint64_t n, uint32_t* bases, uint3
 hipError_t run_pack(const uint8_t* flags, const uint32_t* keys, const uint32_t* values, uint64_t n,
                     uint32_t* tvalues, uint32_t* bases, uint32_t* ckeys, uint32_t* cvalues, uint32_t* d_totals,
                     unsigned long long* clear64, unsigned long long miss, uint32_t* clear32, ScanScratch& sc,
-                    hipStream_t s, uint32_t* host, uint32_t seq) {
+                    hipStream_t s, uint32_t* host, uint32_t seq, PackOrder order) {
     const uint32_t nt = tiles_for(n);
     if (nt > MAX_TILES || (nt == 0 && host)) return hipErrorInvalidValue;
     if (nt == 0) {
@@ -1047,7 +1059,7 @@ hipError_t run_pack(const uint8_t* flags, const uint32_t* keys, const uint32_t* 
     k_pack_tiles<<<nt, 256, 0, s>>>(flags, keys, n, meta);
     k_pack_scan<<<1, 1024, 0, s>>>(meta, nt, d_totals, bases, host, seq);
     k_pack_write<<<nt, 256, 0, s>>>(flags, keys, values, n, meta, tvalues, bases, ckeys, cvalues, clear64, miss,
-                                    clear32);
+                                    clear32, (uint32_t)order, d_totals);
     return hipGetLastError();
 }
 
@@ -1140,26 +1152,28 @@ void launch_ray_sizes(const uint32_t* d_n, uint32_t n_cap, uint32_t leaf, uint32
 constexpr uint32_t ROWSCAN_IN_DOWNSWEEP = 8;
 
 // d_n: device-sized (n and nt are capacities; the kernels read the count)
-template <uint32_t RB>
+template <uint32_t RB, uint32_t ITEMS>
 void radix_pass(const uint32_t* ik, const uint32_t* iv, uint64_t n, uint32_t shift, uint32_t nt, uint32_t* ok,
                 uint32_t* ov, ScanScratch& sc, hipStream_t s, const uint32_t* d_n = nullptr) {
-    k_radix_upsweep<RB><<<nt, 256, 0, s>>>(ik, n, shift, sc.hist.as<uint32_t>(), nt, d_n);
+    uint32_t* hist = sc.hist.as<uint32_t>();
+    uint32_t* totals = sc.digit_totals.as<uint32_t>();
+    k_radix_upsweep<RB, ITEMS><<<nt, 256, 0, s>>>(ik, n, shift, hist, nt, d_n);
     if (nt <= ROWSCAN_IN_DOWNSWEEP && !d_n) {
-        k_radix_downsweep<true, RB><<<nt, 256, 0, s>>>(ik, iv, n, shift, sc.hist.as<uint32_t>(), nt, nullptr, ok, ov,
-                                                       nullptr);
+        k_radix_downsweep<true, RB, ITEMS><<<nt, 256, 0, s>>>(ik, iv, n, shift, hist, nt, nullptr, ok, ov, nullptr);
     } else {
-        k_radix_rowscan<<<1u << RB, 256, 0, s>>>(sc.hist.as<uint32_t>(), nt, sc.digit_totals.as<uint32_t>(), d_n);
-        k_radix_downsweep<false, RB><<<nt, 256, 0, s>>>(ik, iv, n, shift, sc.hist.as<uint32_t>(), nt,
-                                                        sc.digit_totals.as<uint32_t>(), ok, ov, d_n);
+        k_radix_rowscan<<<1u << RB, 256, 0, s>>>(hist, nt, totals, d_n);
+        k_radix_downsweep<false, RB, ITEMS><<<nt, 256, 0, s>>>(ik, iv, n, shift, hist, nt, totals, ok, ov, d_n);
     }
 }
 
 // LSD radix sort of the low `bits` key bits: 8-bit digits, or 9-bit digits
-// where they need fewer passes (17-18 and 25-27 bits).
+// where they need fewer passes (17-18 and 25-27 bits); tiles by the pair count
+// (SMALL_SORT).
 hipError_t run_radix_sort(const uint32_t* keys, const uint32_t* values, uint64_t n, uint32_t bits,
                           uint32_t* out_keys, uint32_t* out_values, ScanScratch& sc, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    uint32_t nt = tiles_for(n);
+    const bool small = n <= SMALL_SORT;
+    const uint32_t nt = small ? (uint32_t)((n + SMALL_SORT_TILE - 1) / SMALL_SORT_TILE) : tiles_for(n);
     if (bits == 0) bits = 1;
     if (bits > 32) bits = 32;
     const uint32_t rb = (bits + 8) / 9 < (bits + 7) / 8 ? 9u : 8u;
@@ -1181,8 +1195,10 @@ hipError_t run_radix_sort(const uint32_t* keys, const uint32_t* values, uint64_t
     }
     for (uint32_t pass = 0; pass < passes; pass++) {
         uint32_t dst = ((passes - 1 - pass) & 1u) ? 0u : 1u;
-        if (rb == 9) radix_pass<9>(ik, iv, n, 9 * pass, nt, bk[dst], bv[dst], sc, s);
-        else radix_pass<8>(ik, iv, n, 8 * pass, nt, bk[dst], bv[dst], sc, s);
+        if (small && rb == 9) radix_pass<9, 4>(ik, iv, n, 9 * pass, nt, bk[dst], bv[dst], sc, s);
+        else if (small) radix_pass<8, 4>(ik, iv, n, 8 * pass, nt, bk[dst], bv[dst], sc, s);
+        else if (rb == 9) radix_pass<9, 16>(ik, iv, n, 9 * pass, nt, bk[dst], bv[dst], sc, s);
+        else radix_pass<8, 16>(ik, iv, n, 8 * pass, nt, bk[dst], bv[dst], sc, s);
         ik = bk[dst];
         iv = bv[dst];
     }
@@ -1207,8 +1223,8 @@ hipError_t run_radix_sort_dev(const uint32_t* keys, const uint32_t* values, uint
     const uint32_t* iv = values;
     for (uint32_t pass = 0; pass < passes; pass++) {
         uint32_t dst = ((passes - 1 - pass) & 1u) ? 0u : 1u;
-        if (rb == 9) radix_pass<9>(ik, iv, n_cap, 9 * pass, nt, bk[dst], bv[dst], sc, s, d_n);
-        else radix_pass<8>(ik, iv, n_cap, 8 * pass, nt, bk[dst], bv[dst], sc, s, d_n);
+        if (rb == 9) radix_pass<9, 16>(ik, iv, n_cap, 9 * pass, nt, bk[dst], bv[dst], sc, s, d_n);
+        else radix_pass<8, 16>(ik, iv, n_cap, 8 * pass, nt, bk[dst], bv[dst], sc, s, d_n);
         ik = bk[dst];
         iv = bv[dst];
     }

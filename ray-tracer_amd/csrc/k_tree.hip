@@ -594,7 +594,7 @@ hipError_t TreeBuild::reserve(uint32_t T) {
         b.take(box, (size_t)T * 32); b.take(blk, (size_t)blocks * 32); b.take(scodes, (size_t)T * 4);
         b.take(sids, (size_t)T * 4); b.take(queue, wide * 4); b.take(count, TREE_LEVELS * 4);
         b.take(codes, (size_t)T * 4); b.take(ids, (size_t)T * 4); b.take(sc.ping_k, (size_t)T * 4);
-        b.take(sc.ping_v, (size_t)T * 4); b.take(sc.hist, (size_t)512 * (tiles_for(T) + 1) * 4);
+        b.take(sc.ping_v, (size_t)T * 4); b.take(sc.hist, sort_hist_bytes(T));
         b.take(sc.digit_totals, 512 * 4); b.take(range, (size_t)T * 8); b.take(child, (size_t)T * 8);
         if (pass) break;
         e = keep.reserve(a.off);

@@ -21,6 +21,32 @@ constexpr uint32_t MAX_TILES = 16384;
 // Exclusive scans up to this length run in one workgroup.
 constexpr uint32_t SMALL_SCAN = 131072;
 
+// Sorts of up to SMALL_SORT pairs run on tiles of 4 items a thread: a digit
+// pass is then one tile's latency, not bandwidth, and a tile of 16 items a
+// thread takes 12 us to rank, one of 4 takes 6 (a frame of 4096 camera rays:
+// 311 -> 277 us).  Beyond it the tiles of 16 fill the chip, and their
+// longer runs per digit write in wider pieces.
+constexpr uint32_t SMALL_SORT_TILE = SCAN_BLOCK * 4;
+constexpr uint32_t SMALL_SORT = 128 * SMALL_SORT_TILE;
+// Digit counts of a sort of up to n pairs (9-bit digits; any smaller sort
+// fits too).
+inline size_t sort_hist_bytes(uint64_t n) {
+    const uint64_t nt = (n + TILE - 1) / TILE + 1, ns = SMALL_SORT / SMALL_SORT_TILE;
+    return (size_t)512 * (nt > ns ? nt : ns) * sizeof(uint32_t);
+}
+
+// What a pass sorts: its packets (chunks of equal keys), expanded afterwards,
+// or its live rays themselves.  Both give the same order (the sort is stable
+// and a packet's rays are neighbours).  Sorting rays drops the four launches of
+// the expansion (34 us of a 100k-ray pass, whatever its size) but moves N pairs
+// a digit pass instead of C.  Up to 2^20 rays that costs less than it saves at
+// any N / C (100k shadow rays 270 -> 220 us; 1080p frame 2.88 -> 2.62 ms); above
+// it, 16 views in one pass of 1.9M rays and N / C = 5 take 8.1 ms sorted as rays
+// and 7.9 as packets, while with N / C < 2 the rays are again the cheaper (1M
+// incoherent rays 802 -> 755 us).
+enum PackOrder : uint32_t { PACK_CHUNKS = 0, PACK_RAYS = 1, PACK_EITHER = 2 };
+__host__ __device__ inline bool sorts_rays(uint32_t N, uint32_t C) { return N <= (1u << 20) || N / 2 <= C; }
+
 inline uint32_t tiles_for(uint64_t n) { return (uint32_t)((n + TILE - 1) / TILE); }
 
 // Sizes of one ray pass kept in device memory (device-sized passes): the
@@ -105,11 +131,13 @@ hipError_t run_compress(const uint32_t* keys, uint64_t n, uint32_t* bases, uint3
 // clear64 (if set) receives `miss` in every slot, clear32 (if set) 0: the pass's
 // per-slot results start cleared.  host (if set, device-visible coherent
 // host memory) receives N and C in host[1], host[2] and then `seq` in host[0]
-// as soon as they are known, ahead of the chunk writes.
+// as soon as they are known, ahead of the chunk writes.  order PACK_RAYS, or
+// PACK_EITHER where sorts_rays(N, C): ckeys / cvalues receive the N live rays'
+// keys and values instead, and tvalues and bases are not written.
 hipError_t run_pack(const uint8_t* flags, const uint32_t* keys, const uint32_t* values, uint64_t n,
                     uint32_t* tvalues, uint32_t* bases, uint32_t* ckeys, uint32_t* cvalues, uint32_t* d_totals,
                     unsigned long long* clear64, unsigned long long miss, uint32_t* clear32, ScanScratch& sc,
-                    hipStream_t s, uint32_t* host = nullptr, uint32_t seq = 0);
+                    hipStream_t s, uint32_t* host = nullptr, uint32_t seq = 0, PackOrder order = PACK_CHUNKS);
 // Exclusive scan of the work-item counts ceil(cand[t] / chunk), t < ntop, with
 // first[ntop] = their total (counts is scratch of ntop + 1 entries); max_cand
 // bounds every cand entry (the scene's cluster count).  zero[0, zero_n) is

@@ -1,0 +1,74 @@
+"""Sorting a pass's rays directly against sorting its packets, and the sort's
+small tiles: the same order, at the edges of the tiles and of the rule that
+picks between the two."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+COUNTERS = ("pass_rays", "pass_chunks", "pass_pairs_top", "pass_pairs_leaf", "pass_ray_tests")
+
+
+def counters(st):
+    return {f: list(getattr(st, f)) for f in COUNTERS}
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 8 * 1024, 8 * 1024 + 1, 128 * 1024, 128 * 1024 + 1])
+@pytest.mark.parametrize("bits", [8, 27, 32])
+def test_sort_tiles(rsh, n, bits):
+    L = rsh.lib()
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n, dtype=np.uint64).astype(np.uint32)
+    keys[: n // 3] = keys[0]            # one long run: a digit that fills whole tiles
+    vals = np.arange(n, dtype=np.uint32)
+    dk, dv = rsh.DeviceArray.from_host(keys), rsh.DeviceArray.from_host(vals)
+    ok, ov = rsh.DeviceArray((n,), np.uint32), rsh.DeviceArray((n,), np.uint32)
+    L.rsh_sort_pairs(dk.ptr, dv.ptr, n, bits, ok.ptr, ov.ptr)
+    assert L.rsh_compat_status() == 0, L.rsh_compat_error()
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(ok.download(), keys[order])
+    np.testing.assert_array_equal(ov.download(), vals[order])
+
+
+@pytest.mark.parametrize("n,runs", [(1, 1), (4097, 50), (1 << 20, 300), ((1 << 20) + 1, 300), ((1 << 20) + 1, 1 << 20)])
+def test_rays_and_packets(rsh, n, runs):
+    """A query's pair and test counts (functions of the sorted order) with the
+    rays sorted (where the rule says so) and with its packets sorted (the order
+    read-back, bit 6), and equal results."""
+    sc = rsh.scenes.config0_scene()
+    cfg = dataclasses.replace(rsh.config.config0(8, 8), cell_bits=4, dir_bits=8).with_scene_bounds(sc)
+    rng = np.random.default_rng(n + runs)
+    o = rng.uniform(sc.bounds_min, sc.bounds_max, (runs, 3))
+    d = rng.normal(size=(runs, 3))
+    rays = np.repeat(np.concatenate([o, d / np.linalg.norm(d, axis=1, keepdims=True)], 1), -(-n // runs), 0)[:n]
+    rays = rays.astype(np.float32)
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        a = e.trace(rays, 0, cfg, flags=2)
+        ca = counters(e.stats)
+        b = e.trace(rays, 0, cfg, flags=2 | 64)
+        assert ca == counters(e.stats)
+        assert ca["pass_rays"][0] == n
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(e.trace(rays, 0, cfg), b)
+    finally:
+        e.close()
+
+
+def test_frame_passes(rsh):
+    """The passes of a frame, whose slots are only partly live."""
+    sc = rsh.scenes.config0_scene()
+    cfg = rsh.config.config0(203, 149).with_scene_bounds(sc)
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        cam = rsh.scenes.config0_camera(203, 149)
+        ca = counters(e.render(cam, cfg, flags=2))
+        pa = e.pixels()
+        assert ca == counters(e.render(cam, cfg, flags=2 | 64))
+        np.testing.assert_array_equal(pa, e.pixels())
+    finally:
+        e.close()

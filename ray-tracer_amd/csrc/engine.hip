@@ -773,13 +773,21 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     level_sizes(N, cfg.leaf, cfg.branch, cfg.depth, counts, offs);
     {
         StageTimer t(L, ST_HIER, timing);
-        if (!presorted)
-            launch_gather(rays, sorted_values, N, psz, kind == 1 ? shadow_pos : nullptr, kind == 1 ? tmax : nullptr,
-                          e->W, e->Lmax, kind == 1 && shadow_pos && cfg.soft_shadows ? 4u : 0u, f4p(L.rec0),
-                          f4p(L.rec1), s, f4p(e->light_pos));
-        launch_hierarchy(f4p(L.rec0), f4p(L.rec1), psz, nullptr, nullptr, N, cfg.leaf, cfg.branch, cfg.depth,
-                         cfg.initial_radius, cfg.initial_spread, cfg.cone_mode, f4p(L.nodes), L.aux.as<float2>(),
-                         counts, offs, s);
+        const float4* pos = kind == 1 ? shadow_pos : nullptr;
+        const float* tm = kind == 1 ? tmax : nullptr;
+        const uint32_t shift = kind == 1 && shadow_pos && cfg.soft_shadows ? 4u : 0u;
+        if (fuses_levels(N, cfg.leaf, cfg.branch, cfg.depth)) {
+            launch_levels(rays, presorted ? nullptr : sorted_values, N, psz, pos, tm, e->W, e->Lmax, shift,
+                          f4p(e->light_pos), cfg.leaf, cfg.branch, cfg.initial_radius, cfg.initial_spread,
+                          cfg.cone_mode, offs[1], f4p(L.rec0), f4p(L.rec1), f4p(L.nodes), L.aux.as<float2>(), s);
+        } else {
+            if (!presorted)
+                launch_gather(rays, sorted_values, N, psz, pos, tm, e->W, e->Lmax, shift, f4p(L.rec0), f4p(L.rec1), s,
+                              f4p(e->light_pos));
+            launch_hierarchy(f4p(L.rec0), f4p(L.rec1), psz, nullptr, nullptr, N, cfg.leaf, cfg.branch, cfg.depth,
+                             cfg.initial_radius, cfg.initial_spread, cfg.cone_mode, f4p(L.nodes), L.aux.as<float2>(),
+                             counts, offs, s);
+        }
         LANE_OK(hipGetLastError());
     }
     if ((flags_mask & 64u) && pass_idx < e->kept.size()) {

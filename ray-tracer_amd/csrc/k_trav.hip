@@ -44,37 +44,47 @@ inline uint32_t grid_for(uint64_t n, uint32_t block, uint32_t cap = 1u << 20) {
 // pixel-light slot), else 0.
 // rays == nullptr (a frame's shadow pass): each ray is recomputed from its
 // slot's surface point and light as k_create_shadow made it (shadow_ray).
-__global__ void __launch_bounds__(256) k_gather(const float* rays, const uint32_t* sorted_values, uint32_t N,
-                                                const PassSizes* ps, const float4* shadow_pos, const float* tmax_in,
-                                                const float4* light_pos, uint32_t W, uint32_t Lmax,
-                                                uint32_t slot_shift, float4* rec0, float4* rec1, FastDiv fw,
-                                                FastDiv fl) {
-    if (ps) N = min(N, ps->N);
-    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < N; p += gridDim.x * blockDim.x) {
-        uint32_t slot = sorted_values[p];
-        v3 o, d;
-        v3 P = mk(0.0f, 0.0f, 0.0f);
-        if (shadow_pos) {
-            const uint32_t i = slot >> slot_shift;
-            const uint32_t qw = fdiv(i, fw);              // l + Lmax y
-            const uint32_t x = i - qw * W, y = fdiv(qw, fl);
-            P = xyz(shadow_pos[(size_t)x + (size_t)y * W]);
-            if (!rays) shadow_ray(P, xyz(light_pos[qw - y * Lmax]), slot_shift != 0u, slot & 15u, o, d);
-        }
-        if (rays) {
-            const float2* r = reinterpret_cast<const float2*>(rays + 6 * (size_t)slot);
-            float2 a = r[0], b = r[1], c = r[2];
-            o = mk(a.x, a.y, b.x); d = mk(b.y, c.x, c.y);
-        }
-        float tmax = 0.0f;
-        if (tmax_in) {
-            tmax = tmax_in[slot];
-        } else if (shadow_pos) {
-            tmax = len(o - P) - EPS * 2.0f;
-        }
-        rec0[p] = f4(o, __uint_as_float(slot));
-        rec1[p] = f4(d, tmax);
+struct GatherParams {
+    const float* rays;
+    const uint32_t* sorted_values;
+    const float4* shadow_pos;
+    const float* tmax_in;
+    const float4* light_pos;
+    uint32_t W, Lmax, slot_shift;
+    FastDiv fw, fl;
+};
+
+__device__ __forceinline__ void gather_ray(const GatherParams& g, uint32_t p, float4& r0, float4& r1) {
+    uint32_t slot = g.sorted_values[p];
+    v3 o, d;
+    v3 P = mk(0.0f, 0.0f, 0.0f);
+    if (g.shadow_pos) {
+        const uint32_t i = slot >> g.slot_shift;
+        const uint32_t qw = fdiv(i, g.fw);              // l + Lmax y
+        const uint32_t x = i - qw * g.W, y = fdiv(qw, g.fl);
+        P = xyz(g.shadow_pos[(size_t)x + (size_t)y * g.W]);
+        if (!g.rays) shadow_ray(P, xyz(g.light_pos[qw - y * g.Lmax]), g.slot_shift != 0u, slot & 15u, o, d);
     }
+    if (g.rays) {
+        const float2* r = reinterpret_cast<const float2*>(g.rays + 6 * (size_t)slot);
+        float2 a = r[0], b = r[1], c = r[2];
+        o = mk(a.x, a.y, b.x); d = mk(b.y, c.x, c.y);
+    }
+    float tmax = 0.0f;
+    if (g.tmax_in) {
+        tmax = g.tmax_in[slot];
+    } else if (g.shadow_pos) {
+        tmax = len(o - P) - EPS * 2.0f;
+    }
+    r0 = f4(o, __uint_as_float(slot));
+    r1 = f4(d, tmax);
+}
+
+__global__ void __launch_bounds__(256) k_gather(GatherParams g, uint32_t N, const PassSizes* ps, float4* rec0,
+                                                float4* rec1) {
+    if (ps) N = min(N, ps->N);
+    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < N; p += gridDim.x * blockDim.x)
+        gather_ray(g, p, rec0[p], rec1[p]);
 }
 
 // ----------------------------------------------------------- hierarchy ----
@@ -154,6 +164,86 @@ __global__ void __launch_bounds__(256) k_levelN(float4* nodes, float2* aux, uint
         nodes[2 * (size_t)(write_off + j)] = sphere;
         nodes[2 * (size_t)(write_off + j) + 1] = cone;
         if (aux) aux[write_off + j] = make_float2(cos_s(cone.w), tan_s(cone.w));
+    }
+}
+
+// Both levels of a depth-2 hierarchy, and with GATHER the sorted records, in
+// one launch: a block of 512 rays makes its records, folds them from LDS into
+// its 512 / leaf lower nodes and those into its 512 / (leaf branch) top nodes
+// (leaf branch divides 512, so no node has rays of two blocks).  What bounds a
+// pass's records and levels is the chain of three launches with a trip through
+// memory between them, not their bytes or arithmetic; 512 rays give the fold
+// of the lower level a whole wave at a fan-out of 8 (the fold is serial in a
+// node, so its lanes are nodes).  LDS rows are padded by one entry in eight:
+// the lanes of a fold read entries `leaf` apart.  Frame of 64x64 277 -> 265 us,
+// of 512x512 384 -> 371; 100k shadow rays 222 -> 210, 1M diffuse 757 -> 742; with
+// the lower nodes in full-size LDS arrays (37 instead of 21 KB) the larger
+// frames lost 2 %, with blocks of 256 rays nothing changed.
+constexpr uint32_t LEVELS_BLOCK = 512;
+__device__ __forceinline__ uint32_t padded(uint32_t i) { return i + (i >> 3); }
+
+template <bool GATHER>
+__global__ void __launch_bounds__(LEVELS_BLOCK) k_levels(GatherParams g, uint32_t N, const PassSizes* ps,
+                                                         uint32_t leaf, uint32_t branch, float r0, float s0,
+                                                         uint32_t mode, uint32_t top_off, float4* rec0, float4* rec1,
+                                                         float4* nodes, float2* aux) {
+    __shared__ float4 s_o[LEVELS_BLOCK + LEVELS_BLOCK / 8];
+    __shared__ float4 s_d[LEVELS_BLOCK + LEVELS_BLOCK / 8];
+    extern __shared__ float4 s_node[];       // lower nodes' spheres, then their cones
+    const uint32_t cap = padded(LEVELS_BLOCK / leaf);
+    if (ps) { N = min(N, ps->N); top_off = ps->offset[1]; }
+    const uint32_t base = blockIdx.x * LEVELS_BLOCK, tid = threadIdx.x;
+    if (base >= N) return;                   // device-sized launches cover capacity
+    const uint32_t n = min(LEVELS_BLOCK, N - base);
+    if (tid < n) {
+        float4 a, b;
+        if (GATHER) {
+            gather_ray(g, base + tid, a, b);
+            rec0[base + tid] = a;
+            rec1[base + tid] = b;
+        } else {
+            a = rec0[base + tid];
+            b = rec1[base + tid];
+        }
+        s_o[padded(tid)] = a;
+        s_d[padded(tid)] = b;
+    }
+    __syncthreads();
+    const uint32_t n0 = (n + leaf - 1) / leaf;
+    if (tid < n0) {
+        const uint32_t f = tid * leaf;
+        const v3 d = xyz(s_d[padded(f)]);
+        float4 sphere = f4(xyz(s_o[padded(f)]), r0);
+        float4 cone = f4(mode == 0 ? d : normalize(d), s0);
+        for (uint32_t i = f + 1; i < min(f + leaf, n); i++) {
+            sphere = sphere_union(sphere, f4(xyz(s_o[padded(i)]), r0));
+            cone = cone0(cone, xyz(s_d[padded(i)]), s0, mode);
+        }
+        const uint32_t j = base / leaf + tid;
+        s_node[padded(tid)] = sphere;
+        s_node[cap + padded(tid)] = cone;
+        nodes[2 * (size_t)j] = sphere;
+        nodes[2 * (size_t)j + 1] = cone;
+        if (aux) aux[j] = make_float2(cos_s(cone.w), tan_s(cone.w));
+    }
+    if (LEVELS_BLOCK / leaf <= 64) {         // the first wave holds every lower node
+        if (tid >= 64) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+        __syncthreads();
+    }
+    const uint32_t n1 = (n0 + branch - 1) / branch;
+    if (tid < n1) {
+        const uint32_t f = tid * branch;
+        float4 sphere = s_node[padded(f)], cone = s_node[cap + padded(f)];
+        for (uint32_t i = f + 1; i < min(f + branch, n0); i++) {
+            sphere = sphere_union(sphere, s_node[padded(i)]);
+            cone = coneN(cone, s_node[cap + padded(i)], mode);
+        }
+        const uint32_t j = top_off + base / (leaf * branch) + tid;
+        nodes[2 * (size_t)j] = sphere;
+        nodes[2 * (size_t)j + 1] = cone;
+        if (aux) aux[j] = make_float2(cos_s(cone.w), tan_s(cone.w));
     }
 }
 
@@ -1457,9 +1547,31 @@ __global__ void __launch_bounds__(256) k_hits_intersect(const float* rays, const
 void launch_gather(const float* rays, const uint32_t* sorted_values, uint32_t N, const PassSizes* ps,
                    const float4* shadow_pos, const float* tmax, uint32_t W, uint32_t Lmax, uint32_t slot_shift,
                    float4* rec0, float4* rec1, hipStream_t s, const float4* light_pos) {
-    if (N) k_gather<<<grid_for(N, 256, 65536), 256, 0, s>>>(rays, sorted_values, N, ps, shadow_pos, tmax, light_pos,
-                                                            W, Lmax, slot_shift, rec0, rec1, fast_div(W),
-                                                            fast_div(Lmax));
+    GatherParams g{rays, sorted_values, shadow_pos, tmax, light_pos, W, Lmax, slot_shift, fast_div(W), fast_div(Lmax)};
+    if (N) k_gather<<<grid_for(N, 256, 65536), 256, 0, s>>>(g, N, ps, rec0, rec1);
+}
+
+// Up to 2^20 rays; beyond, a launch a level fills the chip with whole waves of
+// nodes and leaves the other lane's traversal its LDS (soft shadows, 3.9M rays:
+// 3.124 ms a frame so, 3.143 in one launch).
+bool fuses_levels(uint32_t N, uint32_t leaf, uint32_t branch, uint32_t depth) {
+    return N <= (1u << 20) && depth == 2 && leaf <= LEVELS_BLOCK && branch <= LEVELS_BLOCK && LEVELS_BLOCK % (leaf * branch) == 0;
+}
+
+void launch_levels(const float* rays, const uint32_t* sorted_values, uint32_t N, const PassSizes* ps,
+                   const float4* shadow_pos, const float* tmax, uint32_t W, uint32_t Lmax, uint32_t slot_shift,
+                   const float4* light_pos, uint32_t leaf, uint32_t branch, float r0, float s0, uint32_t mode,
+                   uint32_t top_offset, float4* rec0, float4* rec1, float4* nodes, float2* aux, hipStream_t s) {
+    if (!N) return;
+    GatherParams g{rays, sorted_values, shadow_pos, tmax, light_pos, W, Lmax, slot_shift, fast_div(W), fast_div(Lmax)};
+    const uint32_t blocks = (N - 1) / LEVELS_BLOCK + 1;
+    const uint32_t low = LEVELS_BLOCK / leaf, lds = 2 * (low + low / 8 + 1) * (uint32_t)sizeof(float4);
+    if (sorted_values)
+        k_levels<true><<<blocks, LEVELS_BLOCK, lds, s>>>(g, N, ps, leaf, branch, r0, s0, mode, top_offset, rec0, rec1,
+                                                       nodes, aux);
+    else
+        k_levels<false><<<blocks, LEVELS_BLOCK, lds, s>>>(g, N, ps, leaf, branch, r0, s0, mode, top_offset, rec0, rec1,
+                                                        nodes, aux);
 }
 
 // ps: device-sized (N, counts and offsets are capacities; the kernels read

@@ -281,6 +281,14 @@ void launch_gather(const float* rays, const uint32_t* sorted_values, uint32_t N,
                    const float4* shadow_pos,
                    const float* tmax, uint32_t W, uint32_t Lmax, uint32_t slot_shift, float4* rec0, float4* rec1,
                    hipStream_t s, const float4* light_pos = nullptr);
+// Records (as launch_gather; none where sorted_values is null: rec0 / rec1 hold
+// them) and both levels of the hierarchy in one launch, for the fan-outs that
+// fuses_levels accepts.  top_offset: first node of the upper level.
+bool fuses_levels(uint32_t N, uint32_t leaf, uint32_t branch, uint32_t depth);
+void launch_levels(const float* rays, const uint32_t* sorted_values, uint32_t N, const PassSizes* ps,
+                   const float4* shadow_pos, const float* tmax, uint32_t W, uint32_t Lmax, uint32_t slot_shift,
+                   const float4* light_pos, uint32_t leaf, uint32_t branch, float r0, float s0, uint32_t mode,
+                   uint32_t top_offset, float4* rec0, float4* rec1, float4* nodes, float2* aux, hipStream_t s);
 // Ray queries: key, value (= index) and live flag of n caller rays (float[6n]);
 // segs (optional) places a per-ray segment id at kc.h.segment_shift.
 template <typename F>

@@ -72,3 +72,27 @@ def test_frame_passes(rsh):
         np.testing.assert_array_equal(pa, e.pixels())
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("leaf,branch", [(8, 8), (4, 1), (2, 256), (64, 8), (16, 2), (8, 3)])
+def test_levels(rsh, oracle, leaf, branch):
+    """Records and both hierarchy levels in one launch (fan-outs whose product
+    divides 512; the last pair takes a launch a level), at ray counts about the
+    block's 512, against the oracle bit for bit."""
+    sc = rsh.scenes.config0_scene()
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        for w, h in ((2, 1), (3, 3), (9, 7), (73, 7), (64, 8), (27, 19), (41, 25)):
+            cfg = dataclasses.replace(rsh.config.config0(w, h), leaf=leaf, branch=branch).with_scene_bounds(sc)
+            cam = rsh.scenes.config0_camera(w, h)
+            e.render(cam, cfg, flags=e.KEEP_ORDER)
+            ofr = oracle.render(sc, cam, cfg, keep_order=True, keep_hits=False)
+            for i, op in enumerate(ofr.passes):
+                assert e.stats.pass_rays[i] == op["rays"]
+                if op["rays"]:
+                    g = e.pass_order(i)["nodes"]
+                    np.testing.assert_array_equal(g.view(np.uint32), op["nodes"][:len(g)].view(np.uint32),
+                                                  err_msg=f"{w}x{h}, pass {i}")
+    finally:
+        e.close()

@@ -314,8 +314,9 @@ void launch_hits_intersect(const float* rays, const uint32_t* svalues, const uin
                            const float4* gpos, uint32_t shadow, uint32_t* out, hipStream_t s);
 
 // --- triangle tree (k_tree.hip) ---
-// A four-wide node: per child (lo xyz, word), (hi xyz, -).  Word: node index,
-// or leaf flag | (triangles - 1) << 29 | first record; all ones: no child.
+// A four-wide node: per child (lo xyz, word), (hi xyz, the binary node it was
+// built from).  Word: node index, or leaf flag | (triangles - 1) << 29 | first
+// record; all ones: no child.
 struct TreeNode {
     float4 child[4][2];
 };
@@ -323,7 +324,8 @@ static_assert(sizeof(TreeNode) == 128, "a node is one cache line");
 
 struct TreeBuild {
     DevBuf nodes, records, bounds;                                          // what the traversal reads (parts of keep)
-    DevBuf box, blk, codes, ids, scodes, sids, range, child, queue, count;  // construction (parts of work)
+    // construction (parts of work)
+    DevBuf box, node, size, left, left_count, codes, ids, scodes, sids, queue, count;
     ScanScratch sc;                                                         // the sort's scratch (part of work)
     DevBuf keep, work;
     hipError_t reserve(uint32_t T);

@@ -159,3 +159,36 @@ def test_serving_mix_on_the_soup(engine, rsh):
     for mix in (queries.PRIMARY, queries.DIFFUSE):
         rays, _, _ = queries.make_query(sc, mix, 5003, np.random.default_rng(9))
         check(engine, rsh, sc, rays)
+
+
+@pytest.mark.parametrize("T", [2047, 2048, 2049, 2051, 32768, 32769])
+def test_merge_groups(engine, rsh, T):
+    """Around the triangles of one merging workgroup, and of the sixteen whose
+    clusters the next launch takes."""
+    rng = np.random.default_rng(T)
+    sc = make_scene(rsh, soup(rng, T, size=2.0), 97)
+    check(engine, rsh, sc, rays_at(rng, sc, 501))
+
+
+@pytest.mark.parametrize("kind", ["equal", "nested", "grid", "far"])
+def test_merge_orders(engine, rsh, kind):
+    """Clusters that offer no clear best partner: equal triangles, each inside
+    the next (one pair a round, so the rounds run out), a regular grid, and
+    coordinates whose surfaces overflow."""
+    rng = np.random.default_rng(3)
+    T = 2300
+    if kind == "equal":
+        tris = np.repeat(soup(rng, 1), T, 0)
+    elif kind == "nested":
+        c = soup(rng, 1, size=1.0)
+        mid = c.mean(1, keepdims=True)
+        tris = mid + (c - mid) * (1.006 ** np.arange(T))[:, None, None] * 1e-2
+    elif kind == "grid":
+        g = np.stack(np.meshgrid(np.arange(48), np.arange(48), indexing="ij"), -1).reshape(-1, 2)[:T]
+        base = np.concatenate([g, np.zeros((T, 1))], 1)[:, None] * 2.0 + 50.0
+        tris = base + np.array([[0, 0, 0], [2, 0, 0], [0, 2, 0]])[None]
+    else:
+        tris = soup(rng, T)
+        tris[::3] *= 1e15
+    sc = make_scene(rsh, tris.astype(np.float32), 50)
+    check(engine, rsh, sc, rays_at(rng, sc, 501))

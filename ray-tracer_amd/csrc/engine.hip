@@ -684,6 +684,7 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     if (cfg.algorithm == RSH_CRSH && !dev && !(flags_mask & 64u))
         order = !e->replaying ? PACK_EITHER
                 : sorts_rays(L.plan[L.plan_pos].N, L.plan[L.plan_pos].C) ? PACK_RAYS : PACK_CHUNKS;
+    const bool small = order != PACK_CHUNKS && !all_unique && S > 0 && S <= SMALL_PASS;
     if (all_unique) {
         // hit records cleared: no trim or compression to time
         launch_fill_u64(u64p(closest), cfg.hit_mode == 0 ? MISS64 : (unsigned long long)MISS32, S, s);
@@ -696,7 +697,13 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         const unsigned long long miss = cfg.hit_mode == 0 ? MISS64 : (unsigned long long)MISS32;
         const bool poll = !e->replaying && S > 0;
         // slot flags are bytes; a live slot's value is its index (creation writes no values)
-        LANE_OK(run_pack(u8p(L.flags), u32p(L.keys), nullptr, S, u32p(L.tvalues), u32p(L.bases),
+        if (small)
+            LANE_OK(run_pack_sort(u8p(L.flags), u32p(L.keys), S, sort_bits ? sort_bits : key_bits(cfg),
+                                  u32p(L.svalues), dc, kind == 0 ? u64p(closest) : nullptr, miss,
+                                  kind == 1 ? u32p(closest) : nullptr, s, poll ? L.hsize_dev : nullptr,
+                                  poll ? ++L.hseq : 0u));
+        else
+            LANE_OK(run_pack(u8p(L.flags), u32p(L.keys), nullptr, S, u32p(L.tvalues), u32p(L.bases),
                         u32p(L.ckeys), u32p(L.cvalues), dc, kind == 0 ? u64p(closest) : nullptr, miss,
                         kind == 1 ? u32p(closest) : nullptr, L.sc, s, poll ? L.hsize_dev : nullptr,
                         poll ? ++L.hseq : 0u, order));
@@ -735,6 +742,9 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         StageTimer t(L, ST_SORT, timing);
         LANE_OK(run_radix_sort(u32p(L.keys), u32p(L.values), N, sort_bits ? sort_bits : key_bits(cfg), u32p(L.skeys),
                                u32p(L.svalues), L.sc, s));
+        sorted_values = u32p(L.svalues);
+    } else if (small) {
+        out.C = hc[1];
         sorted_values = u32p(L.svalues);
     } else if (order == PACK_RAYS || (order == PACK_EITHER && sorts_rays(N, hc[1]))) {
         out.C = hc[1];

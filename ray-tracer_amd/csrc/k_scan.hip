@@ -895,6 +895,123 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
     }
 }
 
+// ------------------------------------------------------- a small pass ------
+// Trimming, the packet count and the sort of a pass of up to SMALL_PASS slots
+// in one workgroup, all in LDS: sorted values (slots) of the live rays, the
+// per-slot results cleared, N and C published as by run_pack.  The grid-wide
+// path takes nine launches here, each a launch's latency and gap for a few
+// thousand rays: frame of 64x64 253 -> 217 us, host query of 1000 rays 245 ->
+// 207.  Bound by its barriers and the ballots of the ranking (four digit passes
+// of 16384 pairs: 16 rounds of nine ballots a wave each).
+template <uint32_t ITEMS>
+__global__ void __launch_bounds__(1024) k_pack_sort(const uint8_t* flags, const uint32_t* keys, uint32_t n,
+                                                    uint32_t bits, uint32_t* out_values, unsigned long long* clear64,
+                                                    unsigned long long miss, uint32_t* clear32, uint32_t* totals,
+                                                    uint32_t* host, uint32_t seq) {
+    __shared__ uint32_t sk[1024 * ITEMS];
+    __shared__ uint16_t sv[1024 * ITEMS];
+    __shared__ uint16_t whist[16][512];
+    __shared__ uint32_t start[512];
+    __shared__ uint32_t red[16];
+    const uint32_t tid = threadIdx.x, w = wave_id(), lane = lane_id();
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
+    uint32_t flag[ITEMS];
+#pragma unroll
+    for (uint32_t r = 0; r < ITEMS; r++) {
+        const uint32_t i = (w * ITEMS + r) * 64 + lane;
+        flag[r] = i < n ? flags[i] : 1u;
+        key[r] = i < n ? keys[i] : 0u;          // a dead slot's is not used
+    }
+    for (uint32_t i = tid; i < n; i += 1024) {
+        if (clear64) clear64[i] = miss;
+        if (clear32) clear32[i] = 0u;
+    }
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < ITEMS; r++) {
+        const uint64_t b = __ballot(flag[r] == 0u);
+        rank[r] = mine + (uint32_t)__popcll(b & lt);
+        mine += (uint32_t)__popcll(b);
+    }
+    uint32_t N, C, before;
+    before = block_excl_sum(lane == 0 ? mine : 0u, red, &N);     // of lane 0: the waves before
+    before = (uint32_t)__shfl((int)before, 0, 64);
+#pragma unroll
+    for (uint32_t r = 0; r < ITEMS; r++) {
+        if (flag[r] == 0u) {
+            sk[before + rank[r]] = key[r];
+            sv[before + rank[r]] = (uint16_t)((w * ITEMS + r) * 64 + lane);
+        }
+    }
+    __syncthreads();
+    uint32_t heads = 0;
+    for (uint32_t i = tid; i < N; i += 1024) heads += i == 0 || sk[i] != sk[i - 1] ? 1u : 0u;
+    (void)block_excl_sum(heads, red, &C);
+    if (tid == 0) {
+        totals[0] = N; totals[1] = C;
+        if (host) {
+            host[1] = N;
+            host[2] = C;
+            __threadfence_system();
+            __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    if (N == 0) return;
+    const uint32_t rounds = (N + 1023) / 1024;
+    for (uint32_t shift = 0; shift < bits; shift += 9) {
+        const uint32_t mask = bits - shift < 9 ? (1u << (bits - shift)) - 1u : 511u;
+#pragma unroll
+        for (uint32_t r = 0; r < ITEMS; r++) {
+            const uint32_t i = (w * rounds + r) * 64 + lane;
+            if (r < rounds && i < N) { key[r] = sk[i]; val[r] = sv[i]; }
+        }
+        for (uint32_t i = tid; i < 16 * 512 / 2; i += 1024) reinterpret_cast<uint32_t*>(&whist[0][0])[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < ITEMS; r++) {
+            if (r >= rounds) break;
+            const bool valid = (w * rounds + r) * 64 + lane < N;
+            const uint32_t d = (key[r] >> shift) & mask;
+            uint64_t peers = __ballot(valid);
+#pragma unroll
+            for (uint32_t b = 0; b < 9; b++) {
+                const uint64_t bal = __ballot((d >> b) & 1u);
+                peers &= ((d >> b) & 1u) ? bal : ~bal;
+            }
+            const uint32_t ahead = (uint32_t)__popcll(peers & lt);
+            const uint32_t base = valid ? whist[w][d] : 0u;
+            rank[r] = base + ahead;
+            if (valid && ahead == 0) whist[w][d] = (uint16_t)(base + (uint32_t)__popcll(peers));
+        }
+        __syncthreads();
+        uint32_t sum = 0, all;
+        if (tid < 512) {
+#pragma unroll
+            for (uint32_t q = 0; q < 16; q++) {
+                const uint32_t c = whist[q][tid];
+                whist[q][tid] = (uint16_t)sum;
+                sum += c;
+            }
+        }
+        const uint32_t st = block_excl_sum(sum, red, &all);
+        if (tid < 512) start[tid] = st;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < ITEMS; r++) {
+            const uint32_t i = (w * rounds + r) * 64 + lane;
+            if (r < rounds && i < N) {
+                const uint32_t d = (key[r] >> shift) & mask;
+                const uint32_t at = start[d] + whist[w][d] + rank[r];
+                sk[at] = key[r];
+                sv[at] = (uint16_t)val[r];
+            }
+        }
+        __syncthreads();
+    }
+    for (uint32_t i = tid; i < N; i += 1024) out_values[i] = sv[i];
+}
+
 // --------------------------------------------------------- decompression --
 __global__ void __launch_bounds__(256) k_skeleton(const uint32_t* sizes, const uint32_t* sorted_cvalues, uint64_t C,
                                                   uint32_t* skeleton, const uint32_t* d_c) {
@@ -1044,6 +1161,20 @@ hipError_t run_compress(const uint32_t* keys, uint64_t n, uint32_t* bases, uint3
     return hipGetLastError();
 }
 
+// Radix digits: 8 bits, or 9 where they need fewer passes (17-18 and 25-27 bits).
+static uint32_t digit_bits(uint32_t bits) { return (bits + 8) / 9 < (bits + 7) / 8 ? 9u : 8u; }
+
+hipError_t run_pack_sort(const uint8_t* flags, const uint32_t* keys, uint32_t n, uint32_t bits, uint32_t* out_values,
+                         uint32_t* d_totals, unsigned long long* clear64, unsigned long long miss, uint32_t* clear32,
+                         hipStream_t s, uint32_t* host, uint32_t seq) {
+    if (n == 0 || n > SMALL_PASS) return hipErrorInvalidValue;
+    bits = bits == 0 ? 1u : bits > 32 ? 32u : bits;
+    auto k = n <= 4096 ? k_pack_sort<4> : n <= 8192 ? k_pack_sort<8> : k_pack_sort<16>;
+    const uint32_t rb = digit_bits(bits), sorted = (bits + rb - 1) / rb * rb;      // as run_radix_sort
+    k<<<1, 1024, 0, s>>>(flags, keys, n, sorted < 32 ? sorted : 32u, out_values, clear64, miss, clear32, d_totals, host, seq);
+    return hipGetLastError();
+}
+
 hipError_t run_pack(const uint8_t* flags, const uint32_t* keys, const uint32_t* values, uint64_t n,
                     uint32_t* tvalues, uint32_t* bases, uint32_t* ckeys, uint32_t* cvalues, uint32_t* d_totals,
                     unsigned long long* clear64, unsigned long long miss, uint32_t* clear32, ScanScratch& sc,
@@ -1166,8 +1297,7 @@ void radix_pass(const uint32_t* ik, const uint32_t* iv, uint64_t n, uint32_t shi
     }
 }
 
-// LSD radix sort of the low `bits` key bits: 8-bit digits, or 9-bit digits
-// where they need fewer passes (17-18 and 25-27 bits); tiles by the pair count
+// LSD radix sort of the low `bits` key bits; tiles by the pair count
 // (SMALL_SORT).
 hipError_t run_radix_sort(const uint32_t* keys, const uint32_t* values, uint64_t n, uint32_t bits,
                           uint32_t* out_keys, uint32_t* out_values, ScanScratch& sc, hipStream_t s) {
@@ -1176,7 +1306,7 @@ hipError_t run_radix_sort(const uint32_t* keys, const uint32_t* values, uint64_t
     const uint32_t nt = small ? (uint32_t)((n + SMALL_SORT_TILE - 1) / SMALL_SORT_TILE) : tiles_for(n);
     if (bits == 0) bits = 1;
     if (bits > 32) bits = 32;
-    const uint32_t rb = (bits + 8) / 9 < (bits + 7) / 8 ? 9u : 8u;
+    const uint32_t rb = digit_bits(bits);
     const uint32_t passes = (bits + rb - 1) / rb;
     // Ping-pong so that the final pass lands in out_*.
     uint32_t* bk[2] = {sc.ping_k.as<uint32_t>(), out_keys};
@@ -1213,7 +1343,7 @@ hipError_t run_radix_sort_dev(const uint32_t* keys, const uint32_t* values, uint
     if (nt > MAX_TILES) return hipErrorInvalidValue;
     if (bits == 0) bits = 1;
     if (bits > 32) bits = 32;
-    const uint32_t rb = (bits + 8) / 9 < (bits + 7) / 8 ? 9u : 8u;
+    const uint32_t rb = digit_bits(bits);
     const uint32_t passes = (bits + rb - 1) / rb;
     if (keys == out_keys || values == out_values || keys == out_values || values == out_keys)
         return hipErrorInvalidValue;

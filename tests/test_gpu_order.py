@@ -96,3 +96,49 @@ def test_levels(rsh, oracle, leaf, branch):
                                                   err_msg=f"{w}x{h}, pass {i}")
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 1023, 1025, 4095, 4096, 4097, 8192, 8193, 16383, 16384, 16385])
+@pytest.mark.parametrize("bits", [(4, 8), (3, 4), (4, 9)])
+def test_small_passes(rsh, n, bits):
+    """Passes sorted by one workgroup, at its sizes' edges: the pair and test
+    counts of the packets' path, and equal results; few and many equal keys."""
+    sc = rsh.scenes.config0_scene()
+    cell, dirs = bits
+    cfg = dataclasses.replace(rsh.config.config0(8, 8), cell_bits=cell, dir_bits=dirs).with_scene_bounds(sc)
+    rng = np.random.default_rng(n)
+    o = rng.uniform(sc.bounds_min, sc.bounds_max, (n, 3))
+    d = rng.normal(size=(n, 3))
+    rays = np.concatenate([o, d / np.linalg.norm(d, axis=1, keepdims=True)], 1).astype(np.float32)
+    rays[: n // 2] = rays[0]
+    tmax = np.full(n, 60.0, np.float32)
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        for kind in (0, 1):
+            a = e.trace(rays, kind, cfg, tmax=tmax, flags=2)
+            ca = counters(e.stats)
+            b = e.trace(rays, kind, cfg, tmax=tmax, flags=2 | 64)
+            assert ca == counters(e.stats)
+            np.testing.assert_array_equal(a, b)
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (31, 33), (64, 64), (127, 129), (128, 128)])
+def test_small_frames(rsh, w, h):
+    """Frames whose shadow and reflection passes (partly live) fit one workgroup."""
+    sc = rsh.scenes.config0_scene()
+    cfg = rsh.config.config0(w, h).with_scene_bounds(sc)
+    cam = rsh.scenes.config0_camera(w, h)
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        ca = counters(e.render(cam, cfg, flags=2))
+        pa = e.pixels()
+        assert ca == counters(e.render(cam, cfg, flags=2 | 64))
+        np.testing.assert_array_equal(pa, e.pixels())
+        e.render(cam, cfg)
+        np.testing.assert_array_equal(pa, e.pixels())
+    finally:
+        e.close()

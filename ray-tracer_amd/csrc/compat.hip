@@ -162,7 +162,9 @@ rsh_status reflection_creation(rsh_ctx& c, hipStream_t s, unsigned W, unsigned H
                                unsigned* flags, unsigned* keys, unsigned* values) {
     CTX_OK(need(c, c.g_pos, "bindFragmentPositionArray"));
     CTX_OK(need(c, c.g_nrm, "bindFragmentNormalArray"));
-    launch_create_reflection(c.g_pos, c.g_nrm, c.g_dif ? c.g_dif : c.g_pos, W, H, c.light_max,
+    GBufView g{const_cast<float4*>(c.g_pos), const_cast<float4*>(c.g_nrm),
+               const_cast<float4*>(c.g_dif ? c.g_dif : c.g_pos), nullptr, nullptr, nullptr};
+    launch_create_reflection(g, W, H, c.light_max,
                              single_view(W, H, V(eye)), 0, 0, ref_keys(), reinterpret_cast<float*>(rays), flags, keys,
                              values, s);
     CTX_HIP(hipGetLastError(), "ReflectionRayCreationWrapper");
@@ -326,7 +328,7 @@ rsh_status shadow_coloring(rsh_ctx& c, hipStream_t s, unsigned W, unsigned H, un
         return fail(c, RSH_INVALID_ARG,
                     "ShadowRayColoringWrapper: lightTotal exceeds the bound lights or LIGHT_SOURCE_MAXIMUM");
     GBufView g{const_cast<float4*>(c.g_pos), const_cast<float4*>(c.g_nrm), const_cast<float4*>(c.g_dif),
-               const_cast<float4*>(c.g_spec)};
+               const_cast<float4*>(c.g_spec), nullptr, nullptr};
     launch_shade_primary(g, W, H, c.light_max, Lights{c.light_pos, c.light_col, c.light_int, L},
                          single_view(W, H, V(eye)), sflags, 0u, pixels, s);
     CTX_HIP(hipGetLastError(), "ShadowRayColoringWrapper");

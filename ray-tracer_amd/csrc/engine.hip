@@ -173,7 +173,12 @@ struct rsh_engine {
     std::vector<uint8_t> gsig;         // views + config + scene epoch the graph was captured for
     uint64_t gepoch = 0;               // allocation epoch at capture
     rsh_frame_stats gstats{};          // statistics of the captured frame
-    DevBuf g0[4], gb[2][4];
+    // surface records: positions, normals with the material (GBufView)
+    DevBuf g0[2], gb[2][2];
+    // the material tables of the last frame's records where a scene was loaded
+    // since (a read-back still takes the colours from them)
+    DevBuf old_mat[2];
+    bool framed = false, records_old = false;
 
     // kept passes (flag bit 0), by pass index
     struct Kept {
@@ -239,7 +244,9 @@ inline uint32_t* u32p(const DevBuf& b) { return b.as<uint32_t>(); }
 inline uint8_t* u8p(const DevBuf& b) { return b.as<uint8_t>(); }
 inline unsigned long long* u64p(const DevBuf& b) { return b.as<unsigned long long>(); }
 
-GBufView view(rsh_engine* e, DevBuf* g) { return GBufView{f4p(g[0]), f4p(g[1]), f4p(g[2]), f4p(g[3])}; }
+GBufView view(rsh_engine* e, DevBuf* g) {
+    return GBufView{f4p(g[0]), f4p(g[1]), nullptr, nullptr, f4p(e->mat_dif), f4p(e->mat_spec)};
+}
 
 SceneView scene_view(rsh_engine* e) {
     SceneView s;
@@ -431,7 +438,7 @@ rsh_status ensure_frame(rsh_engine* e, uint32_t W, uint32_t H, uint32_t Lmax, ui
     if (P > e->cap_pixels) {
         HIP_OK(e->rays_b.reserve(P * 24));
         HIP_OK(e->pixels.reserve(P * 4));
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < 2; i++) {
             HIP_OK(e->g0[i].reserve(P * 16)); HIP_OK(e->gb[0][i].reserve(P * 16));
             HIP_OK(e->gb[1][i].reserve(P * 16));
         }
@@ -1019,7 +1026,7 @@ void rsh_engine_destroy(rsh_engine* e) {
     e->tree.release();
     if (e->gexec) (void)hipGraphExecDestroy(e->gexec);
     if (e->graph) (void)hipGraphDestroy(e->graph);
-    for (int i = 0; i < 4; i++) { e->g0[i].release(); e->gb[0][i].release(); e->gb[1][i].release(); }
+    for (int i = 0; i < 2; i++) { e->g0[i].release(); e->gb[0][i].release(); e->gb[1][i].release(); e->old_mat[i].release(); }
     for (auto& k : e->kept) k.release();
     e->frame_rec.release();
     if (e->hrec) (void)hipHostFree(e->hrec);
@@ -1107,6 +1114,12 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     e->T = T; e->K = K; e->M = M; e->L = L;
     HIP_OK(e->tri_pos.reserve((size_t)T * 48)); HIP_OK(e->tri_nrm.reserve((size_t)T * 48));
     HIP_OK(e->tri_mat.reserve((size_t)T * 12));
+    if (e->framed) {       // the last frame's records keep the tables they index
+        std::swap(e->mat_dif, e->old_mat[0]);
+        std::swap(e->mat_spec, e->old_mat[1]);
+        e->framed = false;
+        e->records_old = true;
+    }
     HIP_OK(e->mat_dif.reserve((size_t)M * 16)); HIP_OK(e->mat_spec.reserve((size_t)M * 16));
     HIP_OK(e->light_pos.reserve((size_t)L * 16)); HIP_OK(e->light_col.reserve((size_t)L * 16));
     HIP_OK(e->light_int.reserve((size_t)L * 8));
@@ -1266,6 +1279,8 @@ rsh_status render_frame(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rs
     const bool timing = fl & 4u;
     const bool bs = cfg.bounce_shadows != 0;
     const uint32_t bounces = cfg.bounces < (RSH_MAX_PASSES - 2) / 2 ? cfg.bounces : (RSH_MAX_PASSES - 2) / 2;
+    e->framed = true;
+    e->records_old = false;
     GBufView G0 = view(e, e->g0), GB[2] = {view(e, e->gb[0]), view(e, e->gb[1])};
     float* rays_a = e->rays_a.as<float>();
     float* rays_b = e->rays_b.as<float>();
@@ -1448,7 +1463,7 @@ rsh_status render_frame(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rs
             {
                 StageTimer t(A, ST_CREATE, timing);
                 if (b == 1)
-                    launch_create_reflection(G0.pos, G0.nrm, G0.dif, W, H, Lm, V, cfg.reflect_gate, 1, kc, rays_a,
+                    launch_create_reflection(G0, W, H, Lm, V, cfg.reflect_gate, 1, kc, rays_a,
                                              u8p(A.flags), u32p(A.keys), nullptr, sa);
                 else
                     launch_create_bounce(GB[(b - 1) % 2], W, H, Lm, u64p(e->closest[(b - 1) % 2]), cfg.hit_mode,
@@ -1816,9 +1831,23 @@ rsh_status rsh_engine_read_pixels(rsh_engine* e, uint32_t* host, size_t count) {
 
 rsh_status rsh_engine_read_gbuffer(rsh_engine* e, float* dif, float* spec, float* pos, float* nrm, size_t count) {
     if (!e || count > (size_t)e->W * e->H) return RSH_INVALID_ARG;
-    float* dst[4] = {pos, nrm, dif, spec};
-    for (int i = 0; i < 4; i++)
-        if (dst[i]) HIP_OK(hipMemcpy(dst[i], e->g0[i].p, count * 16, hipMemcpyDeviceToHost));
+    if (pos) HIP_OK(hipMemcpy(pos, e->g0[0].p, count * 16, hipMemcpyDeviceToHost));
+    GBufView g = view(e, e->g0);
+    if (e->records_old) { g.mat_dif = f4p(e->old_mat[0]); g.mat_spec = f4p(e->old_mat[1]); }
+    float* dst[3] = {nrm, dif, spec};
+    if (!count || !(nrm || dif || spec)) return RSH_OK;
+    HIP_OK(hipSetDevice(e->device));
+    float4* out = nullptr;       // not a DevBuf: a captured frame does not use it
+    HIP_OK(hipMalloc(reinterpret_cast<void**>(&out), count * 16));
+    hipError_t err = hipSuccess;
+    for (uint32_t i = 0; i < 3 && err == hipSuccess; i++) {
+        if (!dst[i]) continue;
+        launch_expand_gbuffer(g, i + 1, count, out, e->stream);
+        err = hipMemcpyAsync(dst[i], out, count * 16, hipMemcpyDeviceToHost, e->stream);
+        if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
+    }
+    (void)hipFree(out);
+    HIP_OK(err);
     return RSH_OK;
 }
 

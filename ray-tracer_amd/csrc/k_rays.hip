@@ -182,11 +182,35 @@ __global__ void __launch_bounds__(256) k_create_shadow(const float4* gpos, const
     }
 }
 
+// A surface record's diffuse and specular colour, and its reflection gate.
+__device__ __forceinline__ void colours(const GBufView& g, uint32_t p, float4 n4, float4& Kd, float4& Ks) {
+    if (g.dif) {
+        Kd = g.dif[p]; Ks = g.spec[p];
+    } else {
+        const uint32_t m = __float_as_uint(n4.w);
+        Kd = m ? g.mat_dif[m - 1u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        Ks = m ? g.mat_spec[m - 1u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+}
+__device__ __forceinline__ bool reflects(const GBufView& g, uint32_t p) {
+    if (g.dif) return g.dif[p].w > 0.0f;
+    const uint32_t m = __float_as_uint(g.nrm[p].w);
+    return m && g.mat_dif[m - 1u].w > 0.0f;
+}
+
+__global__ void __launch_bounds__(256) k_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out) {
+    for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (uint64_t)gridDim.x * 256) {
+        const float4 n4 = g.nrm[p];
+        float4 Kd, Ks;
+        colours(g, (uint32_t)p, n4, Kd, Ks);
+        out[p] = plane == 1 ? make_float4(n4.x, n4.y, n4.z, 0.0f) : plane == 2 ? Kd : Ks;
+    }
+}
+
 // RayTracer.cu:742-791; slot x + y*W*Lmax.  gate: only diffuse.w > 0 reflects.
 // mark_gaps: also flag the unused slots between rows when Lmax > 1.
 template <typename F>
-__global__ void __launch_bounds__(256) k_create_reflection(const float4* gpos, const float4* gnrm, const float4* gdif,
-                                                           uint32_t W, uint32_t H, uint32_t Lmax, Views V,
+__global__ void __launch_bounds__(256) k_create_reflection(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, Views V,
                                                            uint32_t gate, uint32_t mark_gaps, KeyCfg kc, float* rays,
                                                            F* flags, uint32_t* keys, uint32_t* values, FastDiv fw) {
     const uint32_t n = W * H;
@@ -197,14 +221,14 @@ __global__ void __launch_bounds__(256) k_create_reflection(const float4* gpos, c
         uint32_t slot = x + y * W * Lmax;
         // the gate first: the surface point and normal of a pixel that does
         // not reflect are never read
-        bool live = !gate || gdif[p].w > 0.0f;
+        bool live = !gate || reflects(g, p);
         v3 P = mk(0.0f, 0.0f, 0.0f);
         if (live) {
-            P = xyz(gpos[p]);
+            P = xyz(g.pos[p]);
             live = dot(P, P) != 0.0f;              // len(P) != 0 without the square root
         }
         if (live) {
-            const v3 N = normalize(xyz(gnrm[p]));
+            const v3 N = normalize(xyz(g.nrm[p]));
             const uint32_t v = view_index(V, s_off, lds, p);
             v3 d = reflect(normalize(P - view_eye(V, v)), normalize(N));
             store_ray(rays, slot, P, d);
@@ -260,7 +284,7 @@ __global__ void __launch_bounds__(256) k_create_bounce(GBufView g, uint32_t W, u
     for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
         const uint32_t y = fdiv(p, fw), x = p - y * W;
         uint32_t slot = x + y * W * Lmax;
-        bool live = rec[slot] != miss && (!gate || g.dif[p].w > 0.0f);
+        bool live = rec[slot] != miss && (!gate || reflects(g, p));
         if (live) {
             v3 o, d;
             load_ray(rays, slot, o, d);
@@ -294,7 +318,8 @@ __global__ void __launch_bounds__(256) k_surface(const float* rays, const unsign
         unsigned long long r = rec[slot];
         if (r == miss) {
             float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            g.pos[p] = z; g.nrm[p] = z; g.dif[p] = z; g.spec[p] = z;
+            g.pos[p] = z; g.nrm[p] = z;
+            if (g.dif) { g.dif[p] = z; g.spec[p] = z; }
             continue;
         }
         uint32_t t = hit_mode == 0 ? (uint32_t)(r & 0xFFFFFFFFull) : (uint32_t)(r & 0x000FFFFFull);
@@ -319,9 +344,11 @@ __global__ void __launch_bounds__(256) k_surface(const float* rays, const unsign
         if (normalize_n) N = normalize(N);
         int32_t m = sc.tri_mat[3 * (size_t)t];
         g.pos[p] = f4(P, 1.0f);
-        g.nrm[p] = f4(N, 0.0f);
-        g.dif[p] = sc.mat_dif[m];
-        g.spec[p] = sc.mat_spec[m];
+        g.nrm[p] = f4(N, g.dif ? 0.0f : __uint_as_float((uint32_t)m + 1u));
+        if (g.dif) {
+            g.dif[p] = sc.mat_dif[m];
+            g.spec[p] = sc.mat_spec[m];
+        }
     }
 }
 
@@ -352,10 +379,12 @@ __global__ void __launch_bounds__(256) k_shade_primary(GBufView g, uint32_t W, u
     for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
         const uint32_t y = fdiv(p, fw), x = p - y * W;
         v3 color = mk(0.0f, 0.0f, 0.0f);
-        v3 P = xyz(g.pos[p]), N = xyz(g.nrm[p]);
+        const float4 n4 = g.nrm[p];
+        v3 P = xyz(g.pos[p]), N = xyz(n4);
         if (dot(P, P) != 0.0f) {                   // len(P) != 0 without the square root
             const v3 eye = view_eye(V, view_index(V, s_off, lds, p));
-            float4 Kd = g.dif[p], Ks = g.spec[p];
+            float4 Kd, Ks;
+            colours(g, p, n4, Kd, Ks);
             for (uint32_t l = 0; l < L.total; l++) {
                 const size_t slot = (size_t)(x + y * W * Lmax) + (size_t)W * l;
                 if (!soft) {
@@ -385,8 +414,10 @@ __global__ void __launch_bounds__(256) k_shade_reflection(GBufView g, uint32_t W
         uint32_t slot = x + y * W * Lmax;
         if (rec[slot] == miss) continue;
         const v3 eye = view_eye(V, view_index(V, s_off, lds, p));
-        v3 P = xyz(g.pos[p]), N = xyz(g.nrm[p]);
-        float4 Kd = g.dif[p], Ks = g.spec[p];
+        const float4 n4 = g.nrm[p];
+        v3 P = xyz(g.pos[p]), N = xyz(n4);
+        float4 Kd, Ks;
+        colours(g, p, n4, Kd, Ks);
         v3 color = mk(0.0f, 0.0f, 0.0f);
         for (uint32_t l = 0; l < L.total; l++) {
             const size_t sl = (size_t)slot + (size_t)W * l;
@@ -569,11 +600,13 @@ void launch_create_shadow(const float4* gpos, const float4* gnrm, uint32_t W, ui
     k_create_shadow<<<grid_for((uint64_t)W * H * Lmax << (soft ? 4 : 0), 256, 65536), 256, 0, s>>>(
         gpos, gnrm, W, H, Lmax, light_pos, kc, V, soft, rays, flags, keys, values, fast_div(W), fast_div(Lmax));
 }
+void launch_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out, hipStream_t s) {
+    if (n) k_expand_gbuffer<<<grid_for(n, 256, 65536), 256, 0, s>>>(g, plane, n, out);
+}
 template <typename F>
-void launch_create_reflection(const float4* gpos, const float4* gnrm, const float4* gdif, uint32_t W, uint32_t H,
-                              uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,
+void launch_create_reflection(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,
                               float* rays, F* flags, uint32_t* keys, uint32_t* values, hipStream_t s) {
-    k_create_reflection<<<grid_for((uint64_t)W * H, 256, 65536), 256, 0, s>>>(gpos, gnrm, gdif, W, H, Lmax, V, gate,
+    k_create_reflection<<<grid_for((uint64_t)W * H, 256, 65536), 256, 0, s>>>(g, W, H, Lmax, V, gate,
                                                                                mark_gaps, kc, rays, flags, keys, values,
                                                                                fast_div(W));
 }
@@ -599,8 +632,8 @@ void launch_create_bounce(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, con
     template void launch_create_shadow<F>(const float4*, const float4*, uint32_t, uint32_t, uint32_t, const float4*, \
                                           KeyCfg, const Views&, uint32_t, float*, F*, uint32_t*, uint32_t*,          \
                                           hipStream_t);                                                              \
-    template void launch_create_reflection<F>(const float4*, const float4*, const float4*, uint32_t, uint32_t,       \
-                                              uint32_t, const Views&, uint32_t, uint32_t, KeyCfg, float*, F*,        \
+    template void launch_create_reflection<F>(GBufView, uint32_t, uint32_t, uint32_t,                               \
+                                              const Views&, uint32_t, uint32_t, KeyCfg, float*, F*,        \
                                               uint32_t*, uint32_t*, hipStream_t);                                    \
     template void launch_create_bounce<F>(GBufView, uint32_t, uint32_t, uint32_t, const unsigned long long*,         \
                                           uint32_t, uint32_t, KeyCfg, const Views&, float*, F*, uint32_t*,           \

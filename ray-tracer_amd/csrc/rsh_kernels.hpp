@@ -85,11 +85,17 @@ inline Views single_view(uint32_t W, uint32_t H, v3 eye, v3 D = v3{0, 0, 1}, v3 
     return v;
 }
 
+// Surface records.  dif and spec null (the engine's own): nrm.w holds the
+// material's index + 1 (0: no surface) and the colours come from the scene's
+// tables, which stay in the caches; with planes of their own they were half of
+// what the surface, shading and ray creation stages moved.
 struct GBufView {
     float4* pos;
     float4* nrm;
     float4* dif;
     float4* spec;
+    const float4* mat_dif;
+    const float4* mat_spec;
 };
 
 // Diagnostic traversal counters are spread over this many slots (summed on
@@ -238,9 +244,10 @@ void launch_create_shadow(const float4* gpos, const float4* gnrm, uint32_t W, ui
                           const float4* light_pos, KeyCfg kc, const Views& V, uint32_t soft, float* rays, F* flags,
                           uint32_t* keys, uint32_t* values, hipStream_t s);
 template <typename F>
-void launch_create_reflection(const float4* gpos, const float4* gnrm, const float4* gdif, uint32_t W, uint32_t H,
-                              uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,
+void launch_create_reflection(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,
                               float* rays, F* flags, uint32_t* keys, uint32_t* values, hipStream_t s);
+// Plane `plane` (1 normals, 2 diffuse, 3 specular) of records without planes.
+void launch_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out, hipStream_t s);
 void launch_create_primary_sorted(const Views& V, uint32_t P, float4* rec0, float4* rec1, hipStream_t s);
 void launch_create_refraction(const float4* gpos, const float4* gnrm, uint32_t W, uint32_t H, uint32_t Lmax,
                               const Views& V, KeyCfg kc, float* rays, uint32_t* flags, uint32_t* keys,

@@ -895,6 +895,13 @@ __global__ void __launch_bounds__(256) k_radix_downsweep(const uint32_t* keys, c
     }
 }
 
+__global__ void k_publish_count(const uint32_t* d, uint32_t* host, uint32_t seq) {
+    if (threadIdx.x != 0) return;
+    host[1] = *d;
+    __threadfence_system();
+    __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ------------------------------------------------------- a small pass ------
 // Trimming, the packet count and the sort of a pass of up to SMALL_PASS slots
 // in one workgroup, all in LDS: sorted values (slots) of the live rays, the
@@ -1159,6 +1166,10 @@ hipError_t run_compress(const uint32_t* keys, uint64_t n, uint32_t* bases, uint3
     k_compress_scatter<<<nt, 256, 0, s>>>(keys, n, tiles, bases, ckeys, cvalues, d_n);
     k_chunk_sizes<<<grid_for(n, 256, 8192), 256, 0, s>>>(bases, d_total, (uint32_t)n, sizes, d_n);
     return hipGetLastError();
+}
+
+void launch_publish_count(const uint32_t* d, uint32_t* host, uint32_t seq, hipStream_t s) {
+    k_publish_count<<<1, 64, 0, s>>>(d, host, seq);
 }
 
 // Radix digits: 8 bits, or 9 where they need fewer passes (17-18 and 25-27 bits).

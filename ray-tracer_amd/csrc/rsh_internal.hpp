@@ -113,6 +113,9 @@ void launch_fill_u64(unsigned long long* p, unsigned long long v, uint64_t n, hi
 hipError_t run_trim(const uint32_t* flags, const uint32_t* keys, const uint32_t* values, uint64_t n,
                     uint32_t* out_keys, uint32_t* out_values, uint32_t* d_total, ScanScratch& sc,
                     hipStream_t s);
+// Device word d to host[1] and then `seq` to host[0] (device-visible coherent
+// host memory), after everything queued on the stream.
+void launch_publish_count(const uint32_t* d, uint32_t* host, uint32_t seq, hipStream_t s);
 // Inclusive scan of flags (the reference's scanArray by-product).
 hipError_t run_inclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, ScanScratch& sc, hipStream_t s);
 // Exclusive scan of u32 values.

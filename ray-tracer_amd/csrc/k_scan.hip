@@ -154,11 +154,15 @@ __global__ void __launch_bounds__(1024) k_unpack_scan(uint32_t* tiles, uint32_t 
 }
 
 // ------------------------------------------------------------- trimming --
+// The live entries are gathered in LDS first, so that a wave stores to
+// neighbouring words (a thread's own run of up to 16 words, stored one by one,
+// touched a line a lane: 7 launches of a 512x512 frame's stages 74 -> 47 us).
 __global__ void __launch_bounds__(256) k_trim_scatter(const uint32_t* flags, const uint32_t* keys,
                                                       const uint32_t* values, uint64_t n,
                                                       const uint32_t* tile_offsets, uint32_t* ok,
                                                       uint32_t* ov) {
     __shared__ uint32_t lds[WAVES];
+    __shared__ uint32_t s_out[TILE];
     const uint64_t base = (uint64_t)blockIdx.x * TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
     uint32_t f[16];
     load16(flags, base, n, f, 1u);
@@ -166,24 +170,37 @@ __global__ void __launch_bounds__(256) k_trim_scatter(const uint32_t* flags, con
 #pragma unroll
     for (int i = 0; i < 16; i++) cnt += f[i] == 0u ? 1u : 0u;
     uint32_t total;
-    uint32_t pos = tile_offsets[blockIdx.x] + block_exclusive_add(cnt, lds, &total);
-    if (cnt == 0) return;
-    uint32_t k[16], v[16];
-    load16(keys, base, n, k, 0u);
-    if (values) load16(values, base, n, v, 0u);
+    const uint32_t first = block_exclusive_add(cnt, lds, &total);
+    if (total == 0) return;
+    const uint32_t at = tile_offsets[blockIdx.x];
+    auto gather = [&](const uint32_t* in, uint32_t* out) {
+        if (cnt) {
+            uint32_t k[16], pos = first;
+            load16(in, base, n, k, 0u);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        if (f[i] == 0u) { ok[pos] = k[i]; if (ov) ov[pos] = v[i]; pos++; }
+            for (int i = 0; i < 16; i++)
+                if (f[i] == 0u) s_out[pos++] = k[i];
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < total; i += blockDim.x) out[at + i] = s_out[i];
+    };
+    gather(keys, ok);
+    if (values && ov) {
+        __syncthreads();
+        gather(values, ov);
     }
 }
 
-// Tile-local scan writer: mode 0 inclusive, mode 1 exclusive.
+// Tile-local scan writer: mode 0 inclusive, mode 1 exclusive.  The tile goes
+// through LDS (rows of 17 words), so that a wave stores to neighbouring words:
+// 8.4M entries 41 us with each thread storing its own 16, 11 so.
 template <int MODE>
 __global__ void __launch_bounds__(256) k_scan_write(const uint32_t* in, uint64_t n, const uint32_t* tile_offsets,
                                                     uint32_t* out, const uint32_t* d_n) {
     __shared__ uint32_t lds[WAVES];
+    __shared__ uint32_t s_out[TILE + TILE / SCAN_ITEMS];
     if (!device_count(d_n, n)) return;
-    const uint64_t base = (uint64_t)blockIdx.x * TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;
+    const uint64_t tile = (uint64_t)blockIdx.x * TILE, base = tile + (uint64_t)threadIdx.x * SCAN_ITEMS;
     uint32_t v[16];
     load16(in, base, n, v, 0u);
     uint32_t s = 0;
@@ -193,11 +210,13 @@ __global__ void __launch_bounds__(256) k_scan_write(const uint32_t* in, uint64_t
     uint32_t run = tile_offsets[blockIdx.x] + block_exclusive_add(s, lds, &total);
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        if (base + i < n) {
-            if (MODE == 0) { run += v[i]; out[base + i] = run; }
-            else { out[base + i] = run; run += v[i]; }
-        }
+        if (MODE == 0) run += v[i];
+        s_out[threadIdx.x * 17 + i] = run;
+        if (MODE != 0) run += v[i];
     }
+    __syncthreads();
+    const uint32_t m = (uint32_t)(n - tile < TILE ? n - tile : TILE);
+    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) out[tile + i] = s_out[i + (i >> 4)];
 }
 
 // ----------------------------------------------------------- compression --

@@ -723,6 +723,151 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
     }
 }
 
+// The same for small passes, a wave per ray: each step takes up to 16 entries
+// off the ray's stack, one to a quad, so a ray that meets hundreds of boxes is a
+// chain of tens of steps instead of hundreds.  It visits boxes that a nearer hit
+// would have spared, on SIMDs that a small pass leaves idle.  Traversal alone, a
+// quad and a wave per ray, 1000 / 8000 / 32000 / 64000 rays: office camera rays 53 /
+// 126 / 131 / 176 us and 18 / 30 / 83 / 165, diffuse rays of the 100k-triangle soup
+// 704 / 905 / 913 / 1021 and 65 / 91 / 216 / 382, of the 2k-triangle room 31 / 38 /
+// 53 / 53 and 14 / 21 / 46 / 77.  The line lies where the last of these meet;
+// camera rays, whose neighbours walk together, meet at half of it (16000 in the
+// room: 26 and 33 us, 32000: 42 and 61).
+constexpr uint32_t WAVE_STACK = 512;
+constexpr uint32_t WAVE_RAYS = 32768, WAVE_CAMERA_RAYS = 16384;
+
+template <int KIND>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace_wave(const TreeParams P) {
+    __shared__ uint32_t s_stack[WAVE_STACK];
+    __shared__ uint16_t s_near[KIND == 0 ? WAVE_STACK : 1];    // entry distance, upper half (rounded down)
+    const uint32_t lane = threadIdx.x, q = lane & 3u, quad = lane >> 2, pos = blockIdx.x;
+    if (pos >= P.N) return;
+    const uint32_t* off = P.level_offset;
+    const float4 r0 = P.rec0[pos], r1 = P.rec1[pos];
+    const v3 d = xyz(r1), o = xyz(r0) + d * EPS;
+    const float dd = dot(d, d);
+    const float tmax = r1.w;
+    const unsigned long long miss = P.hit_mode == 0 ? MISS64 : (unsigned long long)MISS32;
+    const float none = __int_as_float(0x7FC00000);
+    const Slabs S = make_slabs(P, o, d, dd);
+    unsigned long long best = miss;
+    uint32_t best_rec = TREE_EMPTY;
+    bool occluded = false, verify = false;
+    float hi = KIND == 1 ? tmax : none;
+    float lim = KIND == 1 && S.plain ? tmax * 1.002f + S.slack : INFINITY;
+    uint32_t scan = TREE_EMPTY;                // next record of a scan over all triangles
+    uint32_t sp = dd == dd ? 1u : 0u;          // a NaN direction is never hit
+    if (lane == 0) {
+        s_stack[0] = 0u;
+        if (KIND == 0) s_near[0] = 0;
+    }
+    for (;;) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // pushed by one lane, taken by others
+        uint32_t j = TREE_EMPTY;               // the lane's triangle
+        if (sp != 0u) {
+            const uint32_t m = min(min(sp, 16u), (WAVE_STACK - sp) / 3u);
+            if (m == 0u) {                     // full: the ray takes every triangle in turn
+                sp = 0u;
+                scan = 0u;
+                verify = true;
+                best = miss;
+                if (KIND == 0) hi = none;
+                continue;
+            }
+            sp -= m;
+            uint32_t cur = TREE_EMPTY;
+            if (quad < m) {
+                const uint32_t at = sp + m - 1u - quad;
+                const uint32_t c = s_stack[at];
+                if (KIND == 1 || !(__uint_as_float((uint32_t)s_near[at] << 16) > lim)) cur = c;
+            }
+            bool in = false;
+            uint32_t ch = 0u, rank = 0u;
+            float tn = 0.0f;
+            if (!(cur & TREE_IS_LEAF)) {       // whole quads
+                const float4* nb = P.tree[cur].child[q];
+                const float4 a = nb[0], b = nb[1];
+                ch = __float_as_uint(a.w);
+                in = meets(S, a, b, lim, tn);
+                const uint32_t key = in ? (__float_as_uint(tn) & ~3u) | q : 0xFFFFFFFCu | q;
+                rank = (quad_u<QUAD_ROT1>(key) < key ? 1u : 0u) + (quad_u<QUAD_ROT2>(key) < key ? 1u : 0u) +
+                       (quad_u<QUAD_ROT3>(key) < key ? 1u : 0u);
+            } else if (cur != TREE_EMPTY) {
+                const uint32_t n = ((cur >> 29) & 3u) + 1u;
+                if (q < n) j = (cur & 0x1FFFFFFFu) + q;
+            }
+            // the nearest of the topmost entry on top
+            const unsigned long long mask = __ballot(in), from = mask >> (lane & 60u);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // all entries taken
+            if (in) {
+                const uint32_t at = sp + (uint32_t)__popcll(from >> 4) + (uint32_t)__popc((uint32_t)from & 15u) - 1u - rank;
+                s_stack[at] = ch;
+                if (KIND == 0) s_near[at] = (uint16_t)(__float_as_uint(tn) >> 16);
+            }
+            sp += (uint32_t)__popcll(mask);
+        } else if (scan < P.T) {
+            if (scan + lane < P.T) j = scan + lane;
+            scan += 64u;
+        } else {
+            if (KIND == 1 || verify || best_rec == TREE_EMPTY) break;
+            // as in k_tree_trace
+            const float4* rec = P.records + 4 * (size_t)best_rec;
+            if (is_candidate(P, off, pos, __float_as_uint(rec[1].w), __float_as_uint(rec[2].w), rec[0])) break;
+            verify = true;
+            best = miss;
+            hi = none;
+            lim = INFINITY;
+            if (lane == 0) { s_stack[0] = 0u; s_near[0] = 0; }
+            sp = 1u;
+            continue;
+        }
+        unsigned long long mine = best;
+        uint32_t mine_rec = best_rec;
+        if (j != TREE_EMPTY) {
+            const float4* rec = P.records + 4 * (size_t)j;
+            const float4 A = rec[1], B = rec[2], C = rec[3];
+            const float th = ray_triangle(o, d, xyz(A), xyz(B), xyz(C));
+            const uint32_t tri = __float_as_uint(A.w);
+            unsigned long long rc = miss;
+            if (KIND == 1) {
+                if (th > EPS && th < tmax) rc = 0ull;
+            } else if (th > EPS) {
+                rc = pack_hit(th, tri, P.hit_mode);
+            }
+            if (rc < best) {
+                const float4 sph = rec[0];
+                const bool may = P.line_only ? ray_may_hit_sphere(o, d, dd, sph)
+                                             : ray_may_hit_sphere_range(o, d, dd, sph, EPS, hi);
+                if (may && ((KIND == 0 && !verify) || is_candidate(P, off, pos, tri, __float_as_uint(B.w), sph))) {
+                    mine = rc;
+                    mine_rec = j;
+                }
+            }
+        }
+        if (__ballot(mine < best) == 0ull) continue;
+        if (KIND == 1) { occluded = true; break; }
+#pragma unroll
+        for (int x = 32; x > 0; x >>= 1) {
+            const unsigned long long om = __shfl_xor(mine, x, 64);
+            const uint32_t orec = (uint32_t)__shfl_xor((int)mine_rec, x, 64);
+            if (om < mine) { mine = om; mine_rec = orec; }
+        }
+        best = mine;
+        best_rec = mine_rec;
+        if (P.hit_mode == 0) {
+            hi = __uint_as_float((uint32_t)(best >> 32));
+            if (S.plain) lim = hi != hi ? INFINITY : hi * 1.002f + S.slack;
+        }
+    }
+    if (lane != 0u) return;
+    const uint32_t slot = __float_as_uint(r0.w);
+    if (KIND == 1) {
+        if (occluded) P.shadow[slot] = MISS32;
+    } else {
+        P.closest[slot] = best;
+    }
+}
+
 }  // namespace
 
 // One allocation for what the traversal reads, one for the construction.  The I
@@ -814,6 +959,11 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
 
 void launch_tree_trace(const TreeParams& p, hipStream_t s) {
     if (!p.N) return;
+    if (!p.ps && p.N <= (p.line_only ? WAVE_CAMERA_RAYS : WAVE_RAYS)) {
+        if (p.kind == 1) k_tree_trace_wave<1><<<p.N, 64, 0, s>>>(p);
+        else k_tree_trace_wave<0><<<p.N, 64, 0, s>>>(p);
+        return;
+    }
     if (p.kind == 1) k_tree_trace<1><<<grid_for(p.N, 16), 64, 0, s>>>(p);
     else k_tree_trace<0><<<grid_for(p.N, 16), 64, 0, s>>>(p);
 }

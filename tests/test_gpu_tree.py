@@ -192,3 +192,51 @@ def test_merge_orders(engine, rsh, kind):
         tris[::3] *= 1e15
     sc = make_scene(rsh, tris.astype(np.float32), 50)
     check(engine, rsh, sc, rays_at(rng, sc, 501))
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 32769])
+def test_wave_and_quad(engine, rsh, n):
+    """A wave per ray up to 32768 rays and a quad per ray beyond: scenes and
+    rays outside the ordinary on both sides of the line."""
+    rng = np.random.default_rng(n)
+    s = 0.5 ** np.repeat(np.arange(9), 40)[:, None, None]
+    nested = (50.0 + 100.0 * s * (np.asarray([[0.1, 0.1, 0.1], [1.0, 0.1, 0.2], [0.1, 1.0, 0.3]])
+                                  + 0.01 * rng.random((360, 3, 3)))).astype(np.float32)
+    for tris in (soup(rng, 513), nested, np.repeat(soup(rng, 1), 300, 0)):
+        sc = make_scene(rsh, tris, 30)
+        rays = rays_at(rng, sc, n)
+        rays[0:64, 3:] *= 1e6
+        rays[128:192, 3:] = np.eye(3, dtype=np.float32)[rng.integers(3, size=64)]
+        rays[256:264, 3:] = 0.0
+        rays[264:272, 3:] = np.nan
+        rays[280:288, 0] = np.nan
+        rays[296:304, 3:] *= 1e-20
+        rays[312:320, :3] *= 1e16
+        check(engine, rsh, sc, rays)
+        if len(tris) == 513:
+            check(engine, rsh, sc, rays, hit_mode=1)
+            check(engine, rsh, sc, rays, algorithm=1)
+
+
+def test_wave_stack_full(engine, rsh):
+    """Equal boxes by the thousand: a ray's stack fills and it takes every
+    triangle in turn."""
+    rng = np.random.default_rng(4)
+    sc = make_scene(rsh, np.repeat(soup(rng, 1), 20_000, 0), 500)
+    rays = rays_at(rng, sc, 64)
+    rays[:32, 3:] = (sc.tri_pos[:3, :3].mean(0) - rays[:32, :3])
+    check(engine, rsh, sc, rays)
+
+
+@pytest.mark.parametrize("w,h", [(127, 129), (128, 128), (145, 113)])
+def test_wave_camera_passes(engine, rsh, w, h):
+    """Camera passes on both sides of their line (16384 rays)."""
+    sc = rsh.scenes.config0_scene()
+    cfg = rsh.config.config0(w, h).with_scene_bounds(sc)
+    engine.load_scene(sc)
+    cam = rsh.scenes.config0_camera(w, h)
+    engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+    got = [engine.pass_hits(i) for i in range(engine.stats.pass_count)]
+    engine.render(cam, dataclasses.replace(cfg, traversal_prefilter=1), flags=engine.KEEP_PASSES)
+    for i, g in enumerate(got):
+        np.testing.assert_array_equal(g, engine.pass_hits(i))

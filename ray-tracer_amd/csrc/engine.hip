@@ -132,6 +132,7 @@ struct rsh_engine {
     DevBuf tri_pos, tri_nrm, tri_mat, mat_dif, mat_spec, light_pos, light_col, light_int;
     DevBuf tri_sphere, tri_mt, obj_sphere, obj_range;
     TreeBuild tree;                    // triangle tree of the automatic traversal
+    bool has_tree = false;             // built for the loaded scene
     std::vector<float> host_light_pos;   // float4[L] as loaded
     // cluster level: CLUSTER consecutive triangles of one object per cluster
     uint32_t NC = 0;
@@ -834,7 +835,7 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     // The automatic traversal walks the triangle tree; a caller that counts
     // the reference's tests or picks a kernel, a work split or a pre-test gets
     // the kernels these belong to.
-    if (!counting && cfg.traversal_kernel == 0 && cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 &&
+    if (e->has_tree && !counting && cfg.traversal_kernel == 0 && cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 &&
         cfg.traversal_splits == 0) {
         TreeParams q{};
         q.tree = e->tree.nodes.as<TreeNode>(); q.records = f4p(e->tree.records); q.bounds = u32p(e->tree.bounds);
@@ -1180,8 +1181,21 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     HIP_OK(hipMemcpyAsync(e->cl_base.p, base.data(), (size_t)K * 4, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(e->all_list.p, ident.data(), (size_t)K * 16, hipMemcpyHostToDevice, st));
     build_clusters(e, st);
-    HIP_OK(e->tree.reserve(T));
-    HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
+    // A scene too large for the tree (its 29-bit record places, or its memory)
+    // is traced by the kernels that test every candidate.
+    e->has_tree = T <= TREE_MAX_TRIANGLES;
+    if (e->has_tree) {
+        const hipError_t r = e->tree.reserve(T);
+        if (r == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            e->tree.release();
+            e->has_tree = false;
+        } else {
+            HIP_OK(r);
+        }
+    }
+    if (e->has_tree)
+        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
     e->orig_ready = false;
@@ -1961,7 +1975,8 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
     HIP_OK(hipMemcpy2DAsync(e->obj_sphere.p, 16, e->sph_tmp.p, 24, 16, K, hipMemcpyDeviceToDevice, st));
     launch_triangle_prep(f4p(e->tri_pos), T, f4p(e->tri_sphere), f4p(e->tri_mt), st);
     build_clusters(e, st);
-    HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
+    if (e->has_tree)
+        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
     drop_graph(e);

@@ -914,7 +914,7 @@ void TreeBuild::release() {
 
 hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
                             hipStream_t s) {
-    if (T == 0 || T > (1u << 29) || K == 0) return hipErrorInvalidValue;
+    if (T == 0 || T > TREE_MAX_TRIANGLES || K == 0) return hipErrorInvalidValue;
     float4* bx = box.as<float4>();
     uint32_t* bd = bounds.as<uint32_t>();
     k_tree_clear<<<1, 64, 0, s>>>(bd);

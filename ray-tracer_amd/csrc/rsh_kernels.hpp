@@ -329,6 +329,8 @@ struct TreeNode {
 };
 static_assert(sizeof(TreeNode) == 128, "a node is one cache line");
 
+constexpr uint32_t TREE_MAX_TRIANGLES = 1u << 29;      // places in a child word
+
 struct TreeBuild {
     DevBuf nodes, records, bounds;                                          // what the traversal reads (parts of keep)
     // construction (parts of work)

@@ -22,13 +22,14 @@ Beside the headline it measures, on the same GPU:
   "office_obj", "cornell_obj" (with --office / --cornell)
               the reference's thesis scenes read from its model files.
 
-Prints one JSON line.  "roofline" describes the dominant kernel, the fused
-traversal (k_traverse64, one launch per pass): its launch durations come from
+Prints one JSON line.  "roofline" describes the dominant kernel, the
+traversal (k_tree_trace, one launch per pass): its launch durations come from
 HIP events recorded around every traversal launch of three frames rendered
 with serial passes (the timed frames run the shadow passes concurrently with
 the reflection chain, so their launches share the GPU); its algorithmic FLOPs
 from one extra frame with the traversal
-counters on (pair and test counts are deterministic); its HBM traffic from the
+counters on (the reference's pair and test counts, which are deterministic); its
+own VALU instructions from the rocprofv3 summary committed under profiles/; its HBM traffic from the
 rocprofv3 FETCH_SIZE / WRITE_SIZE summary committed under profiles/.
 "cpu_baseline" is the C++ oracle on a band of rows of the same frame.
 
@@ -52,7 +53,10 @@ PEAK_HBM_GBS = 8000.0
 PEAK_FP32_TFLOPS = 157.3
 FLOP_NODE_TEST = 25      # SphereNodeIntersection, RayTracer.cu:283-298
 FLOP_RAY_TEST = 46       # RayTriangleIntersection full path, RayTracer.cu:257-280
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_traverse64_atrium1080p_traffic.txt")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_tree_trace_atrium1080p_traffic.txt")
+VALU_FILE = os.path.join(ROOT, "profiles", "k_tree_trace_atrium1080p_valu.txt")
+# one wave64 instruction per SIMD every 4 cycles: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz
+PEAK_VALU_TLANES = 256 * 4 * 16 * 2.4e9 / 1e12
 
 
 def parse():
@@ -95,11 +99,11 @@ def parse():
                          "average over the serial frames the roofline times")
     ap.add_argument("--trav-traffic", nargs=4, default=None,
                     metavar=("FETCH_CSV", "WRITE_CSV", "COPY_FETCH_CSV", "COPY_WRITE_CSV"),
-                    help="(no GPU) HBM traffic per k_traverse64 launch from rocprofv3 FETCH_SIZE / WRITE_SIZE runs "
+                    help="(no GPU) HBM traffic per k_tree_trace launch from rocprofv3 FETCH_SIZE / WRITE_SIZE runs "
                          "of this bench (--steps 1 --warmup 0, frame legs only), scaled by the same counters on "
                          "--copy-probe 512")
     ap.add_argument("--trav-valu", default="", metavar="SQ_CSV",
-                    help="(no GPU) SQ counters per k_traverse64 launch of the first serial frame")
+                    help="(no GPU) SQ counters per k_tree_trace launch of the first serial frame")
     ap.add_argument("--out", default="")
     return ap.parse_args()
 
@@ -122,6 +126,17 @@ def traffic_per_launch():
     try:
         with open(TRAFFIC_FILE) as f:
             m = re.search(r"^traffic_bytes_per_launch\s*=\s*([0-9.eE+]+)", f.read(), re.M)
+        return float(m.group(1)) if m else None
+    except OSError:
+        return None
+
+
+def valu_per_frame():
+    """VALU wave instructions of the traversal kernel per frame of this
+    workload, from the committed rocprofv3 summary (None when it is absent)."""
+    try:
+        with open(VALU_FILE) as f:
+            m = re.search(r"^VALU instructions per frame: ([0-9.eE+]+)", f.read(), re.M)
         return float(m.group(1)) if m else None
     except OSError:
         return None
@@ -221,7 +236,7 @@ def hsc_figure(passes, stages, cfg, name):
 
 
 HSC_KERNELS = ("k_create_primary_sorted", "k_create_shadow", "k_create_reflection", "k_create_bounce",
-               "k_pack_tiles", "k_pack_scan", "k_pack_write", "k_radix_upsweep", "k_radix_rowscan",
+               "k_pack_sort", "k_pack_tiles", "k_pack_scan", "k_pack_write", "k_radix_upsweep", "k_radix_rowscan",
                "k_radix_downsweep", "k_unpack_sizes", "k_unpack_scan", "k_unpack_offsets", "k_unpack_expand")
 HSC_PROFILES = {"frame": "hsc_atrium1080p_frame.txt", "office": "hsc_office_64views.txt",
                 "atrium": "hsc_atrium_64views.txt"}
@@ -292,7 +307,7 @@ def _kernel_base(name):
 
 def trav_summary(a):
     """--trav-summary: the kernel table of a rocprofv3 --stats run of this
-    bench (frame legs only), the k_traverse64 launches grouped by frame in
+    bench (frame legs only), the k_tree_trace launches grouped by frame in
     start order, and their average over the three serial frames with
     traversal timers, which the roofline's avg_launch_ms times with HIP
     events.  Frames in a run: --warmup warm-up, --steps timed, one eager
@@ -314,22 +329,22 @@ def trav_summary(a):
     launches = []
     with open(trace_csv) as f:
         for r in csv.DictReader(f):
-            if "k_traverse64" in r["Kernel_Name"]:
+            if "k_tree_trace" in r["Kernel_Name"]:
                 launches.append((int(r["Start_Timestamp"]), (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e6))
     launches.sort()
     counts, first = _frame_layout(len(launches), a.steps, a.warmup)
     frames = _split_frames(launches, counts)
     print()
-    print("k_traverse64<8, MODE> per launch (ms), one row per frame, in start order")
+    print("k_tree_trace<KIND> per launch (ms), one row per frame, in start order")
     for i, fr in enumerate(frames):
         tag = "  <- serial, traversal timers" if first <= i < first + 3 else ""
         print("  " + " ".join(f"{d:6.2f}" for _, d in fr) + f"   sum {sum(d for _, d in fr):5.2f}{tag}")
-    serial = [sum(d for _, d in ps) for fr in frames[first:first + 3] for ps in _passes_of(fr)]
+    serial = [d for fr in frames[first:first + 3] for _, d in fr]
     print()
-    print(f"k_traverse64 average launch: {sum(d for _, d in launches) / max(len(launches), 1):.3f} ms over "
+    print(f"k_tree_trace average launch: {sum(d for _, d in launches) / max(len(launches), 1):.3f} ms over "
           f"{len(launches)} launches")
-    print(f"k_traverse64 time per traced pass over the 3 serial frames with traversal timers (the camera pass's "
-          f"two launches together): {sum(serial) / max(len(serial), 1):.3f} ms ({len(serial)} passes)")
+    print(f"k_tree_trace time per traced pass over the 3 serial frames with traversal timers: "
+          f"{sum(serial) / max(len(serial), 1):.3f} ms ({len(serial)} passes)")
 
 
 def _counter_rows(path, kernel=None):
@@ -353,16 +368,14 @@ FRAME_PASSES = len(PASS_NAMES)
 
 
 def _frame_layout(n_launches, steps, warmup):
-    """k_traverse64 launches per frame of a bench run (the --no-* legs off)
+    """k_tree_trace launches per frame of a bench run (the --no-* legs off)
     and the index of its first serial frame with traversal timers.  Frames,
     in order: --warmup warm-up, --steps timed, one eager frame recorded for
     the graph, 1 + --steps graph replays, 3 serial frames with traversal
-    timers, 3 with stage timers, 1 with counters.  The camera pass runs as
-    two launches when it goes front to back (every frame but the counting
-    one), so the other frames have 8 or 9 launches alike."""
-    frames = warmup + steps + 1 + (1 + steps) + 3 + 3 + 1
-    per = (n_launches - FRAME_PASSES) // (frames - 1)
-    return [per] * (frames - 1) + [FRAME_PASSES], warmup + 2 * steps + 2
+    timers, 3 with stage timers (the last one, with counters, runs the kernel
+    that tests every candidate)."""
+    frames = warmup + steps + 1 + (1 + steps) + 3 + 3
+    return [n_launches // frames] * frames, warmup + 2 * steps + 2
 
 
 def _split_frames(items, counts):
@@ -373,28 +386,20 @@ def _split_frames(items, counts):
     return out
 
 
-def _passes_of(frame):
-    """A frame's launches grouped by pass: a front-to-back camera pass's two
-    launches together, then one launch per pass."""
-    if len(frame) == FRAME_PASSES + 1:
-        return [frame[0:2]] + [[x] for x in frame[2:]]
-    return [[x] for x in frame]
-
-
 def _first_serial_frame(dispatches, steps=1, warmup=0):
-    """The k_traverse64 dispatches of the first serial frame with traversal
+    """The k_tree_trace dispatches of the first serial frame with traversal
     timers of a bench run (frame order as in trav_summary), grouped by pass
     in pass order: primary, then shadow and reflection passes alternating
     (in the timed frames the two lanes' launches interleave differently)."""
     d = sorted(dispatches)
     counts, first = _frame_layout(len(d), steps, warmup)
-    return _passes_of(_split_frames(d, counts)[first])
+    return [[x] for x in _split_frames(d, counts)[first]]
 
 
 def trav_traffic(a):
     fetch_csv, write_csv, cf_csv, cw_csv = a.trav_traffic
-    fv, _ = _counter_rows(fetch_csv, "k_traverse64")
-    wv, _ = _counter_rows(write_csv, "k_traverse64")
+    fv, _ = _counter_rows(fetch_csv, "k_tree_trace")
+    wv, _ = _counter_rows(write_csv, "k_tree_trace")
     cfv, _ = _counter_rows(cf_csv, "copyBuffer")
     cwv, _ = _counter_rows(cw_csv, "copyBuffer")
     copy_kib = 512 * 1024
@@ -408,7 +413,7 @@ def trav_traffic(a):
     print()
     fd = _first_serial_frame(fv)
     wd = _first_serial_frame(wv)
-    print("per pass (KiB as counted; the camera pass's two launches summed), the first serial frame of the run:")
+    print("per pass (KiB as counted), the first serial frame of the run:")
     print(f"{'pass':10s} {'FETCH_KiB':>12s} {'WRITE_KiB':>12s} {'scaled_MB':>12s}")
     tf = tw = 0.0
     for name, df, dw in zip(PASS_NAMES, fd, wd):
@@ -424,12 +429,11 @@ def trav_traffic(a):
 
 
 def trav_valu(a):
-    vals, _ = _counter_rows(a.trav_valu, "k_traverse64")
+    vals, _ = _counter_rows(a.trav_valu, "k_tree_trace")
     d = _first_serial_frame(vals)
     keys = ["SQ_WAVES", "SQ_INSTS_VALU", "SQ_INSTS_SALU", "SQ_INSTS_LDS", "SQ_INSTS_VMEM", "SQ_WAVE_CYCLES",
             "SQ_BUSY_CYCLES", "SQ_ACTIVE_INST_VALU"]
-    print("Counters summed over the chip per pass (the first serial frame of the run, passes in order; the camera "
-          "pass's two launches summed).")
+    print("Counters summed over the chip per pass (the first serial frame of the run, passes in order).")
     print(f"{'pass':10s} {'waves':>10s} {'VALU_insts':>12s} {'SALU_insts':>12s} {'LDS_insts':>12s} "
           f"{'VMEM_insts':>12s} {'VALU/wave':>10s}")
     tot = 0.0
@@ -911,13 +915,21 @@ def main():
     flops_frame = FLOP_RAY_TEST * n_tests + FLOP_NODE_TEST * (n_top + cfg.branch * n_surv)
     avg_launch_ms = trav_ms / trav_launches if trav_launches else 0.0
     flops_launch = flops_frame / passes_per_frame if passes_per_frame else 0.0
-    achieved = flops_launch / (avg_launch_ms * 1e-3) / 1e12 if avg_launch_ms > 0 else 0.0
+    reference = flops_launch / (avg_launch_ms * 1e-3) / 1e12 if avg_launch_ms > 0 else 0.0
+    valu = valu_per_frame()
+    achieved = (valu * 64 / (avg_launch_ms * passes_per_frame * 1e-3) / 1e12
+                if valu and avg_launch_ms > 0 and passes_per_frame else 0.0)
     roof = {"bound": "valu",
-            "kernel": "k_traverse64<8, MODE> (fused traversal + intersection; one launch per pass, two for the "
-                      "front-to-back camera pass)",
-            "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
-            "frac": achieved / PEAK_FP32_TFLOPS, "traffic": traffic_per_launch(),
-            "avg_launch_ms": avg_launch_ms, "per": "traced pass (the camera pass's two launches together)",
+            "kernel": "k_tree_trace<KIND>, k_tree_trace_wave<KIND> (tree traversal + intersection + the candidates' "
+                      "node tests; one launch per pass)",
+            "achieved": achieved, "peak": PEAK_VALU_TLANES, "unit": "T lane instructions/s",
+            "frac": achieved / PEAK_VALU_TLANES, "traffic": traffic_per_launch(),
+            "valu_instructions_per_frame": valu,
+            "reference_tflops": reference,
+            "note": "achieved is the kernel's own VALU instruction rate (counts from the committed profile); "
+                    "reference_tflops is the reference's algorithmic work (its pair and ray tests, most of which the "
+                    "tree never runs) per second",
+            "avg_launch_ms": avg_launch_ms, "per": "traced pass",
             "passes_per_frame": passes_per_frame,
             "flops_per_launch": flops_launch}
     hsc = hsc_figure(passes, stages, cfg, "frame")

@@ -266,7 +266,10 @@ rsh_status rsh_engine_read_pixels(rsh_engine* e, uint32_t* host_rgba, size_t cou
  * (flag bit 3) first waits for a pending copy. */
 rsh_status rsh_engine_read_pixels_async(rsh_engine* e, uint32_t* host_rgba, size_t count);
 rsh_status rsh_engine_wait_pixels(rsh_engine* e);
-/* Primary G-buffer: diffuse, specular, position, normal, each float4[W*H]. */
+/* Primary G-buffer: diffuse, specular, position, normal, each float4[W*H].
+ * Of the last frame that completed, with its scene's colours also after another
+ * scene was loaded; RSH_INVALID_ARG where that frame has fewer pixels than
+ * count, or a call with more rays than its buffers held has replaced them. */
 rsh_status rsh_engine_read_gbuffer(rsh_engine* e, float* host_dif, float* host_spec,
                                    float* host_pos, float* host_nrm, size_t count);
 /* Per-slot records of pass i (closest: exact or reference packing; shadow:

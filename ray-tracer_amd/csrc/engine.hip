@@ -176,10 +176,15 @@ struct rsh_engine {
     rsh_frame_stats gstats{};          // statistics of the captured frame
     // surface records: positions, normals with the material (GBufView)
     DevBuf g0[2], gb[2][2];
-    // the material tables of the last frame's records where a scene was loaded
-    // since (a read-back still takes the colours from them)
+    // Pixels of the last completed frame whose records still stand in g0.  None
+    // before a frame, after one that failed, and once a larger call has
+    // reallocated the buffers: their contents then index no material.
+    size_t records = 0;
+    // the material tables of those records, and their length, where a scene was
+    // loaded since (a read-back still takes the colours from them)
     DevBuf old_mat[2];
-    bool framed = false, records_old = false;
+    uint32_t old_M = 0;
+    bool records_old = false;
 
     // kept passes (flag bit 0), by pass index
     struct Kept {
@@ -437,6 +442,7 @@ rsh_status ensure_frame(rsh_engine* e, uint32_t W, uint32_t H, uint32_t Lmax, ui
         e->cap_shadow_slots = Ss;
     }
     if (P > e->cap_pixels) {
+        e->records = 0;
         HIP_OK(e->rays_b.reserve(P * 24));
         HIP_OK(e->pixels.reserve(P * 4));
         for (int i = 0; i < 2; i++) {
@@ -1112,15 +1118,15 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     }
     HIP_OK(hipSetDevice(e->device));
     const uint32_t T = s->triangle_total, K = s->object_total, M = s->material_total, L = s->light_total;
+    if (e->records && !e->records_old) {       // the last frame's records keep the tables they index
+        std::swap(e->mat_dif, e->old_mat[0]);
+        std::swap(e->mat_spec, e->old_mat[1]);
+        e->old_M = e->M;
+        e->records_old = true;
+    }
     e->T = T; e->K = K; e->M = M; e->L = L;
     HIP_OK(e->tri_pos.reserve((size_t)T * 48)); HIP_OK(e->tri_nrm.reserve((size_t)T * 48));
     HIP_OK(e->tri_mat.reserve((size_t)T * 12));
-    if (e->framed) {       // the last frame's records keep the tables they index
-        std::swap(e->mat_dif, e->old_mat[0]);
-        std::swap(e->mat_spec, e->old_mat[1]);
-        e->framed = false;
-        e->records_old = true;
-    }
     HIP_OK(e->mat_dif.reserve((size_t)M * 16)); HIP_OK(e->mat_spec.reserve((size_t)M * 16));
     HIP_OK(e->light_pos.reserve((size_t)L * 16)); HIP_OK(e->light_col.reserve((size_t)L * 16));
     HIP_OK(e->light_int.reserve((size_t)L * 8));
@@ -1293,8 +1299,10 @@ rsh_status render_frame(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rs
     const bool timing = fl & 4u;
     const bool bs = cfg.bounce_shadows != 0;
     const uint32_t bounces = cfg.bounces < (RSH_MAX_PASSES - 2) / 2 ? cfg.bounces : (RSH_MAX_PASSES - 2) / 2;
-    e->framed = true;
-    e->records_old = false;
+    if (!e->replaying) {
+        e->records = 0;
+        e->records_old = false;
+    }
     GBufView G0 = view(e, e->g0), GB[2] = {view(e, e->gb[0]), view(e, e->gb[1])};
     float* rays_a = e->rays_a.as<float>();
     float* rays_b = e->rays_b.as<float>();
@@ -1531,6 +1539,7 @@ rsh_status render_frame(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rs
     }
     if (e->replaying) return RSH_OK;     // under stream capture: no synchronisation
     HIP_OK(hipStreamSynchronize(sa));
+    e->records = P;
     if (st && (timing || (fl & 16u))) {
         for (Lane& l : e->lane)
             for (auto& t : l.timed) {
@@ -1621,6 +1630,8 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
     const std::vector<uint8_t> sig = signature(!(e->gexec && e->gdev));
     if (e->gexec && sig == e->gsig && alloc_epoch().load() == e->gepoch) {
         HIP_OK(hipSetDevice(e->device));
+        e->records = 0;
+        e->records_old = false;
         if (e->gdev)
             HIP_OK(hipMemcpyAsync(e->views_d.p, hv, (size_t)nv * sizeof(ViewDesc), hipMemcpyHostToDevice, e->stream));
         HIP_OK(hipGraphLaunch(e->gexec, e->stream));
@@ -1633,6 +1644,7 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
             drop_graph(e);
             return render_frame(e, hv, nv, cfg, 0, st);
         }
+        e->records = (size_t)P;
         if (st) {
             *st = e->gstats;
             st->graph_replayed = 1;
@@ -1845,18 +1857,23 @@ rsh_status rsh_engine_read_pixels(rsh_engine* e, uint32_t* host, size_t count) {
 
 rsh_status rsh_engine_read_gbuffer(rsh_engine* e, float* dif, float* spec, float* pos, float* nrm, size_t count) {
     if (!e || count > (size_t)e->W * e->H) return RSH_INVALID_ARG;
+    float* dst[3] = {nrm, dif, spec};
+    if (!count || !(pos || nrm || dif || spec)) return RSH_OK;
+    if (count > e->records) {
+        e->err = "read_gbuffer: no completed frame holds this many surface records";
+        return RSH_INVALID_ARG;
+    }
     if (pos) HIP_OK(hipMemcpy(pos, e->g0[0].p, count * 16, hipMemcpyDeviceToHost));
+    if (!(nrm || dif || spec)) return RSH_OK;
     GBufView g = view(e, e->g0);
     if (e->records_old) { g.mat_dif = f4p(e->old_mat[0]); g.mat_spec = f4p(e->old_mat[1]); }
-    float* dst[3] = {nrm, dif, spec};
-    if (!count || !(nrm || dif || spec)) return RSH_OK;
     HIP_OK(hipSetDevice(e->device));
     float4* out = nullptr;       // not a DevBuf: a captured frame does not use it
     HIP_OK(hipMalloc(reinterpret_cast<void**>(&out), count * 16));
     hipError_t err = hipSuccess;
     for (uint32_t i = 0; i < 3 && err == hipSuccess; i++) {
         if (!dst[i]) continue;
-        launch_expand_gbuffer(g, i + 1, count, out, e->stream);
+        launch_expand_gbuffer(g, e->records_old ? e->old_M : e->M, i + 1, count, out, e->stream);
         err = hipMemcpyAsync(dst[i], out, count * 16, hipMemcpyDeviceToHost, e->stream);
         if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
     }

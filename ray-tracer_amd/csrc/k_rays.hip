@@ -198,9 +198,11 @@ __device__ __forceinline__ bool reflects(const GBufView& g, uint32_t p) {
     return m && g.mat_dif[m - 1u].w > 0.0f;
 }
 
-__global__ void __launch_bounds__(256) k_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out) {
+__global__ void __launch_bounds__(256) k_expand_gbuffer(GBufView g, uint32_t materials, uint32_t plane, uint64_t n,
+                                                        float4* out) {
     for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < n; p += (uint64_t)gridDim.x * 256) {
-        const float4 n4 = g.nrm[p];
+        float4 n4 = g.nrm[p];
+        if (__float_as_uint(n4.w) > materials) n4.w = 0.0f;
         float4 Kd, Ks;
         colours(g, (uint32_t)p, n4, Kd, Ks);
         out[p] = plane == 1 ? make_float4(n4.x, n4.y, n4.z, 0.0f) : plane == 2 ? Kd : Ks;
@@ -600,8 +602,8 @@ void launch_create_shadow(const float4* gpos, const float4* gnrm, uint32_t W, ui
     k_create_shadow<<<grid_for((uint64_t)W * H * Lmax << (soft ? 4 : 0), 256, 65536), 256, 0, s>>>(
         gpos, gnrm, W, H, Lmax, light_pos, kc, V, soft, rays, flags, keys, values, fast_div(W), fast_div(Lmax));
 }
-void launch_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out, hipStream_t s) {
-    if (n) k_expand_gbuffer<<<grid_for(n, 256, 65536), 256, 0, s>>>(g, plane, n, out);
+void launch_expand_gbuffer(GBufView g, uint32_t materials, uint32_t plane, uint64_t n, float4* out, hipStream_t s) {
+    if (n) k_expand_gbuffer<<<grid_for(n, 256, 65536), 256, 0, s>>>(g, materials, plane, n, out);
 }
 template <typename F>
 void launch_create_reflection(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,

@@ -246,8 +246,9 @@ void launch_create_shadow(const float4* gpos, const float4* gnrm, uint32_t W, ui
 template <typename F>
 void launch_create_reflection(GBufView g, uint32_t W, uint32_t H, uint32_t Lmax, const Views& V, uint32_t gate, uint32_t mark_gaps, KeyCfg kc,
                               float* rays, F* flags, uint32_t* keys, uint32_t* values, hipStream_t s);
-// Plane `plane` (1 normals, 2 diffuse, 3 specular) of records without planes.
-void launch_expand_gbuffer(GBufView g, uint32_t plane, uint64_t n, float4* out, hipStream_t s);
+// Plane `plane` (1 normals, 2 diffuse, 3 specular) of records without planes;
+// a record's index beyond the `materials` of the tables gives black.
+void launch_expand_gbuffer(GBufView g, uint32_t materials, uint32_t plane, uint64_t n, float4* out, hipStream_t s);
 void launch_create_primary_sorted(const Views& V, uint32_t P, float4* rec0, float4* rec1, hipStream_t s);
 void launch_create_refraction(const float4* gpos, const float4* gnrm, uint32_t W, uint32_t H, uint32_t Lmax,
                               const Views& V, KeyCfg kc, float* rays, uint32_t* flags, uint32_t* keys,

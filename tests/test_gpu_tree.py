@@ -240,3 +240,33 @@ def test_wave_camera_passes(engine, rsh, w, h):
     engine.render(cam, dataclasses.replace(cfg, traversal_prefilter=1), flags=engine.KEEP_PASSES)
     for i, g in enumerate(got):
         np.testing.assert_array_equal(g, engine.pass_hits(i))
+
+
+def tiles(n):
+    """A floor of n x n tiles of one unit, two triangles each."""
+    g = np.stack(np.meshgrid(np.arange(n), np.arange(n), indexing="ij"), -1).reshape(-1, 1, 2).astype(np.float64)
+    g = np.insert(g, 1, 0.0, axis=2)
+    return np.concatenate([g + np.array([[0, 0, 0], [1, 0, 0], [0, 0, 1]]),
+                           g + np.array([[1, 0, 1], [0, 0, 1], [1, 0, 0]])])
+
+
+@pytest.mark.parametrize("n", [1501, 32783])
+@pytest.mark.parametrize("away", [0.0, 2e4, 3e5, 1e6, 1e9])
+def test_scenes_far_from_the_origin(engine, rsh, n, away):
+    """Small scenes and their rays translated, for the wave and the quad kernel.
+    The reference is the kernel with the pre-tests (traversal_prefilter 2): that
+    far out a triangle's sphere, rounded to its coordinates, need not hold the
+    triangle, and the pre-tests take it at its word, as the tree does."""
+    rng = np.random.default_rng(int(away))
+    for tris in (tiles(10), soup(rng, 400, spread=10.0, size=1.0) - 50.0, soup(rng, 2000, spread=100.0)):
+        sc = make_scene(rsh, (tris + away * np.array([1.0, -0.7, 0.4])).astype(np.float32), 50)
+        rays = rays_at(rng, sc, n)
+        cfg = qcfg(rsh, sc)
+        engine.load_scene(sc)
+        tmax = np.full(n, 60.0, np.float32)
+        for kind in (0, 1):
+            got = engine.trace(rays, kind, cfg, tmax=tmax)
+            want = engine.trace(rays, kind, dataclasses.replace(cfg, traversal_prefilter=2), tmax=tmax)
+            np.testing.assert_array_equal(got, want)
+            if away <= 3e5:
+                assert (want != (np.uint64(0xFFFFFFFFFFFFFFFF) if kind == 0 else 0)).sum() > n // 10

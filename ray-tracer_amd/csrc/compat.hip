@@ -18,12 +18,12 @@
 //    overrunning them (the reference has no guard, RayTracer.cu:2788).
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <string>
 
 #include "../../include/rsh.h"
 #include "../../include/rsh_ctx.h"
 #include "../../include/rsh_engine.h"
+#include "host_words.hpp"
 #include "rsh_kernels.hpp"
 
 using namespace rsh;
@@ -45,13 +45,13 @@ struct rsh_ctx {
     DevBuf dtotal;       // uint32[16]: counts of the stages given no device word
     DevBuf psz;          // PassSizes of a hierarchy over a device ray count
     uint64_t scratch_items = 0;
-    uint32_t* hword = nullptr;      // coherent page-locked words k_publish_count writes: seq, count
-    uint32_t* hword_dev = nullptr;  // their device address
+    HostWords hword;     // coherent page-locked words k_publish_count writes: seq, count
     uint32_t hseq = 0;
     void release() {
         sc.release(); dtotal.release(); psz.release(); scratch_items = 0;
-        if (hword) (void)hipHostFree(hword);
-        hword = hword_dev = nullptr;
+        if (hword.host) (void)hipHostFree(hword.host);
+        hword = HostWords{};
+        hseq = 0;                   // the next words start cleared
     }
 };
 
@@ -94,28 +94,24 @@ rsh_status ensure_scratch(rsh_ctx& c, uint64_t n) {
 // all of them).
 rsh_status read_count(rsh_ctx& c, hipStream_t s, const uint32_t* d, uint32_t* h, const char* what) {
     if (!h) return RSH_OK;
-    if (!c.hword) {
-        uint32_t* p = nullptr;
-        CTX_HIP(hipHostMalloc(reinterpret_cast<void**>(&p), 64, hipHostMallocCoherent | hipHostMallocMapped), what);
-        std::memset(p, 0, 64);
-        c.hword = p;
-        CTX_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&c.hword_dev), p, 0), what);
-        c.hseq = 0;
-    }
+    CTX_HIP(acquire_words(c.hword, 64,
+                          [](void** p, size_t n) { return hipHostMalloc(p, n, hipHostMallocCoherent | hipHostMallocMapped); },
+                          [](void** d, void* p) { return hipHostGetDevicePointer(d, p, 0); },
+                          [](void* p) { return hipHostFree(p); }), what);
     const uint32_t seq = ++c.hseq;
-    launch_publish_count(d, c.hword_dev, seq, s);
+    launch_publish_count(d, c.hword.dev, seq, s);
     CTX_HIP(hipGetLastError(), what);
-    for (uint32_t spin = 1; __atomic_load_n(c.hword, __ATOMIC_ACQUIRE) != seq; spin++) {
+    for (uint32_t spin = 1; __atomic_load_n(c.hword.host, __ATOMIC_ACQUIRE) != seq; spin++) {
         if (spin % 4096u == 0) {
             // errors surface here; a stream that has ended has written the word
             const hipError_t r = hipStreamQuery(s);
-            if (r == hipSuccess && __atomic_load_n(c.hword, __ATOMIC_ACQUIRE) != seq)
+            if (r == hipSuccess && __atomic_load_n(c.hword.host, __ATOMIC_ACQUIRE) != seq)
                 CTX_HIP(hipErrorUnknown, what);
             if (r != hipSuccess && r != hipErrorNotReady) CTX_HIP(r, what);
         }
         __builtin_ia32_pause();
     }
-    *h = __atomic_load_n(c.hword + 1, __ATOMIC_RELAXED);
+    *h = __atomic_load_n(c.hword.host + 1, __ATOMIC_RELAXED);
     return RSH_OK;
 }
 

@@ -353,6 +353,14 @@ int rsh_selfcheck_rcp(int device, uint64_t* tested, uint64_t* mismatches);
  * block_ms > wait_ms), RSH_HIP_ERROR when the stream went idle first. */
 rsh_status rsh_selfcheck_wait_deadline(uint32_t wait_ms, uint32_t block_ms, uint32_t* elapsed_ms);
 
+/* Self-check of the triangle tree's traversal (no counterpart in the reference;
+ * used by the test suite): from now on this engine's automatic passes walk the
+ * tree with one kernel whatever their size (walk 1: four lanes a ray, 2: a wave a
+ * ray) or do without the tree as a scene too large for it does (3); 0 goes back
+ * to the rules of size.  small_stack: ray stacks of a few entries, so that most
+ * rays take the path of a full one.  Results are the same in every mode. */
+rsh_status rsh_selfcheck_tree_walk(rsh_engine* e, uint32_t walk, uint32_t small_stack);
+
 /* Device memory helpers (plain HIP calls, for callers without a HIP runtime
  * binding of their own). */
 void* rsh_device_alloc(size_t bytes);

@@ -133,6 +133,7 @@ struct rsh_engine {
     DevBuf tri_sphere, tri_mt, obj_sphere, obj_range;
     TreeBuild tree;                    // triangle tree of the automatic traversal
     bool has_tree = false;             // built for the loaded scene
+    uint32_t tree_walk = WALK_AUTO, tree_small_stack = 0;   // a test's (rsh_selfcheck_tree_walk)
     std::vector<float> host_light_pos;   // float4[L] as loaded
     // cluster level: CLUSTER consecutive triangles of one object per cluster
     uint32_t NC = 0;
@@ -841,8 +842,8 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     // The automatic traversal walks the triangle tree; a caller that counts
     // the reference's tests or picks a kernel, a work split or a pre-test gets
     // the kernels these belong to.
-    if (e->has_tree && !counting && cfg.traversal_kernel == 0 && cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 &&
-        cfg.traversal_splits == 0) {
+    if (e->has_tree && e->tree_walk != WALK_NONE && !counting && cfg.traversal_kernel == 0 &&
+        cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 && cfg.traversal_splits == 0) {
         TreeParams q{};
         q.tree = e->tree.nodes.as<TreeNode>(); q.records = f4p(e->tree.records); q.bounds = u32p(e->tree.bounds);
         q.nodes = f4p(L.nodes); q.aux = L.aux.as<float2>();
@@ -853,6 +854,7 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         q.obj_sphere = f4p(e->obj_sphere); q.obj_range = e->obj_range.as<uint4>();
         q.algorithm = cfg.algorithm; q.kind = kind; q.hit_mode = cfg.hit_mode;
         q.line_only = RSH_CAMERA_LINE_ONLY && camera && kind == 0 ? 1u : 0u;
+        q.walk = e->tree_walk; q.small_stack = e->tree_small_stack;
         q.closest = u64p(closest); q.shadow = u32p(closest);       // by kind
         StageTimer t(L, ST_PASS_TRAVERSE + (int)pass_idx, trav_timing);
         launch_tree_trace(q, s);
@@ -1819,6 +1821,14 @@ rsh_status rsh_engine_trace(rsh_engine* e, const float* rays, const float* tmax,
             if (t.first >= ST_PASS_TRAVERSE) st->pass_traverse_ms[0] += ms;
         }
     }
+    return RSH_OK;
+}
+
+rsh_status rsh_selfcheck_tree_walk(rsh_engine* e, uint32_t walk, uint32_t small_stack) {
+    if (!e || walk > WALK_NONE) return RSH_INVALID_ARG;
+    e->tree_walk = walk;
+    e->tree_small_stack = small_stack ? 1u : 0u;
+    drop_graph(e);
     return RSH_OK;
 }
 

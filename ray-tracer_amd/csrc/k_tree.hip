@@ -502,7 +502,7 @@ __global__ void __launch_bounds__(256) k_tree_records(EmitArgs A, const uint32_t
 // (k_traverse64) with its culling and work list, traversal alone: the frame's
 // 8 passes 4.77 -> 1.84 ms, a query of 1M diffuse rays 9.18 -> 0.52 ms, one of
 // 100k shadow rays 0.54 -> 0.12 ms.
-constexpr uint32_t STACK = 48;
+constexpr uint32_t STACK = 48, SMALL_STACK = 6;       // the latter for the tests of a full stack
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t quad_u(uint32_t x) {
@@ -583,10 +583,10 @@ __device__ __forceinline__ bool meets(const Slabs& s, float4 lo, float4 hi, floa
     return !(tn > tf) && __float_as_uint(lo.w) != TREE_EMPTY;
 }
 
-template <int KIND>
+template <int KIND, uint32_t CAP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace(const TreeParams P) {
-    __shared__ uint32_t s_stack[STACK][16];
-    __shared__ uint16_t s_near[KIND == 0 ? STACK : 1][16];     // entry distance, upper half (rounded down)
+    __shared__ uint32_t s_stack[CAP][16];
+    __shared__ uint16_t s_near[KIND == 0 ? CAP : 1][16];     // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, ray = lane >> 2;
     const uint32_t* off = P.ps ? P.ps->offset : P.level_offset;
     // Workgroups go to the 8 XCDs in turn; 64 neighbours (1024 sorted rays) stay
@@ -636,7 +636,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
             // rank of the lane's child among the hit ones, nearest first
             const uint32_t rank = (quad_u<QUAD_ROT1>(key) < key ? 1u : 0u) + (quad_u<QUAD_ROT2>(key) < key ? 1u : 0u) +
                                   (quad_u<QUAD_ROT3>(key) < key ? 1u : 0u);
-            const bool full = sp + n > STACK;  // no ray of a scene of ordinary depth
+            const bool full = sp + n > CAP;    // no ray of a scene of ordinary depth
             if (in && !full) {
                 const uint32_t at = sp + n - 1u - rank;
                 s_stack[at][ray] = ch;
@@ -739,13 +739,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
 // 53 / 53 and 14 / 21 / 46 / 77.  The line lies where the last of these meet;
 // camera rays, whose neighbours walk together, meet at half of it (16000 in the
 // room: 26 and 33 us, 32000: 42 and 61).
-constexpr uint32_t WAVE_STACK = 512;
+constexpr uint32_t WAVE_STACK = 512, SMALL_WAVE_STACK = 16;
 constexpr uint32_t WAVE_RAYS = 32768, WAVE_CAMERA_RAYS = 16384;
 
-template <int KIND>
+template <int KIND, uint32_t CAP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace_wave(const TreeParams P) {
-    __shared__ uint32_t s_stack[WAVE_STACK];
-    __shared__ uint16_t s_near[KIND == 0 ? WAVE_STACK : 1];    // entry distance, upper half (rounded down)
+    __shared__ uint32_t s_stack[CAP];
+    __shared__ uint16_t s_near[KIND == 0 ? CAP : 1];    // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, quad = lane >> 2, pos = blockIdx.x;
     if (pos >= P.N) return;
     const uint32_t* off = P.level_offset;
@@ -771,7 +771,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // pushed by one lane, taken by others
         uint32_t j = TREE_EMPTY;               // the lane's triangle
         if (sp != 0u) {
-            const uint32_t m = min(min(sp, 16u), (WAVE_STACK - sp) / 3u);
+            const uint32_t m = min(min(sp, 16u), (CAP - sp) / 3u);
             if (m == 0u) {                     // full: the ray takes every triangle in turn
                 sp = 0u;
                 scan = 0u;
@@ -965,13 +965,14 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
 
 void launch_tree_trace(const TreeParams& p, hipStream_t s) {
     if (!p.N) return;
-    if (!p.ps && p.N <= (p.line_only ? WAVE_CAMERA_RAYS : WAVE_RAYS)) {
-        if (p.kind == 1) k_tree_trace_wave<1><<<p.N, 64, 0, s>>>(p);
-        else k_tree_trace_wave<0><<<p.N, 64, 0, s>>>(p);
-        return;
-    }
-    if (p.kind == 1) k_tree_trace<1><<<grid_for(p.N, 16), 64, 0, s>>>(p);
-    else k_tree_trace<0><<<grid_for(p.N, 16), 64, 0, s>>>(p);
+    const bool small = p.N <= (p.line_only ? WAVE_CAMERA_RAYS : WAVE_RAYS);
+    const bool wave = !p.ps && (p.walk == WALK_WAVE || (p.walk != WALK_QUAD && small));
+    auto kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, WAVE_STACK> : k_tree_trace_wave<0, WAVE_STACK>)
+                       : (p.kind == 1 ? k_tree_trace<1, STACK> : k_tree_trace<0, STACK>);
+    if (p.small_stack)
+        kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, SMALL_WAVE_STACK> : k_tree_trace_wave<0, SMALL_WAVE_STACK>)
+                      : (p.kind == 1 ? k_tree_trace<1, SMALL_STACK> : k_tree_trace<0, SMALL_STACK>);
+    kernel<<<wave ? p.N : grid_for(p.N, 16), 64, 0, s>>>(p);
 }
 
 }  // namespace rsh

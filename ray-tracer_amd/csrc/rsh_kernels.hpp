@@ -345,6 +345,10 @@ struct TreeBuild {
     void release();
 };
 
+// How a pass is traced: by the rules of its size, or as a test asks (the tree
+// with one kernel at every size; without the tree).
+enum TreeWalk : uint32_t { WALK_AUTO = 0, WALK_QUAD = 1, WALK_WAVE = 2, WALK_NONE = 3 };
+
 struct TreeParams {
     const TreeNode* tree;
     const float4* records;        // [4T] triangles in tree order
@@ -360,6 +364,7 @@ struct TreeParams {
     const float4* obj_sphere;
     const uint4* obj_range;
     uint32_t algorithm, kind, hit_mode, line_only;
+    uint32_t walk, small_stack;   // a test's (rsh_selfcheck_tree_walk)
     unsigned long long* closest;  // kind 0: every traced ray's record is written
     uint32_t* shadow;             // kind 1: MISS32 where occluded
 };

@@ -270,3 +270,97 @@ def test_scenes_far_from_the_origin(engine, rsh, n, away):
             np.testing.assert_array_equal(got, want)
             if away <= 3e5:
                 assert (want != (np.uint64(0xFFFFFFFFFFFFFFFF) if kind == 0 else 0)).sum() > n // 10
+
+
+# Both traversal kernels at sizes of either's choosing (rsh_selfcheck_tree_walk):
+# above, passes of up to 32768 rays walk a wave per ray only.
+QUAD, WAVE, NO_TREE = 1, 2, 3
+
+
+@pytest.fixture
+def walk(engine):
+    def use(kernel, small_stack=False):
+        assert engine.L.rsh_selfcheck_tree_walk(engine.h, kernel, int(small_stack)) == 0
+    yield use
+    use(0)
+
+
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 8, 9, 63, 65, 513, 2047, 2049, 4099, 32769])
+def test_quad_scene_sizes(engine, rsh, walk, T):
+    rng = np.random.default_rng(T)
+    walk(QUAD)
+    sc = make_scene(rsh, soup(rng, T, size=2.0), 7)
+    check(engine, rsh, sc, rays_at(rng, sc, 1501))
+
+
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 31, 64, 65, 1025, 1040])
+def test_quad_ray_counts(engine, rsh, walk, n):
+    rng = np.random.default_rng(n)
+    sc = make_scene(rsh, soup(rng, 777), 50)
+    walk(QUAD)
+    check(engine, rsh, sc, rays_at(rng, sc, n))
+
+
+@pytest.mark.parametrize("kernel,n", [(QUAD, 2003), (WAVE, 40_001)])
+@pytest.mark.parametrize("variant", [dict(algorithm=1), dict(hit_mode=1), dict(depth=1), dict(depth=3, branch=4),
+                                     dict(depth=4, leaf=4, branch=3), dict(leaf=32, branch=2), dict(key_mode=0),
+                                     dict(triangle_batch=512), dict(cone_mode=0)])
+def test_options_in_both_kernels(engine, rsh, walk, kernel, n, variant):
+    rng = np.random.default_rng(3)
+    sc = make_scene(rsh, soup(rng, 3001), 64)
+    walk(kernel)
+    check(engine, rsh, sc, rays_at(rng, sc, n), **variant)
+
+
+@pytest.mark.parametrize("kernel", [QUAD, WAVE])
+def test_outside_the_ordinary_in_both_kernels(engine, rsh, walk, kernel):
+    walk(kernel)
+    test_scenes_outside_the_ordinary(engine, rsh)
+    test_rays_outside_the_ordinary(engine, rsh)
+    for kind in ("equal", "nested", "grid", "far"):
+        test_merge_orders(engine, rsh, kind)
+    test_serving_mix_on_the_soup(engine, rsh)
+    test_moved_objects(engine, rsh)
+
+
+@pytest.mark.parametrize("kernel", [QUAD, WAVE])
+@pytest.mark.parametrize("variant", [dict(), dict(hit_mode=1), dict(algorithm=1)])
+def test_full_stacks(engine, rsh, walk, kernel, variant):
+    """Stacks of a few entries.  In the scene of equal triangles every box of
+    the tree is the same, so a ray that meets one meets all, and three levels
+    (more than 64 triangles) fill either stack: it then takes every triangle in
+    turn.  The others fill it for some rays."""
+    rng = np.random.default_rng(4)
+    one = soup(rng, 1)
+    for tris in (np.repeat(one, 300, 0), soup(rng, 3001), soup(rng, 400, size=30.0)):
+        sc = make_scene(rsh, tris, 50)
+        rays = rays_at(rng, sc, 1003)
+        rays[:64, 3:] = sc.tri_pos[:3, :3].mean(0) - rays[:64, :3]      # through the first triangle
+        walk(kernel, small_stack=True)
+        want = check(engine, rsh, sc, rays, **variant)
+        if len(tris) == 300:
+            assert want[:64].any()
+    walk(kernel, small_stack=True)
+    test_moved_objects(engine, rsh)
+
+
+def test_frames_without_the_tree(engine, rsh, walk):
+    """A scene too large for the tree: the automatic traversal's other kernels
+    (front-to-back camera pass, work list, ray masks) on the full-size atrium
+    frame, against the tree's frame."""
+    sc = rsh.scenes.config2_scene()
+    cfg = rsh.config.config2().with_scene_bounds(sc)
+    cam = rsh.scenes.config2_camera(cfg.width, cfg.height)
+    engine.load_scene(sc)
+    engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+    modes = list(engine.stats.pass_mode[:engine.stats.pass_count])
+    got = [engine.pass_hits(i) for i in range(engine.stats.pass_count)]
+    px = engine.pixels()
+    walk(NO_TREE)
+    engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+    assert modes == [3] * len(modes) and 3 not in engine.stats.pass_mode[:engine.stats.pass_count]
+    np.testing.assert_array_equal(px, engine.pixels())
+    for i, g in enumerate(got):
+        np.testing.assert_array_equal(g, engine.pass_hits(i))
+    check(engine, rsh, rsh.scenes.soup_scene(triangles=5000),
+          queries.make_query(rsh.scenes.soup_scene(triangles=5000), queries.DIFFUSE, 5003, np.random.default_rng(1))[0])

@@ -133,6 +133,7 @@ struct rsh_engine {
     DevBuf tri_sphere, tri_mt, obj_sphere, obj_range;
     TreeBuild tree;                    // triangle tree of the automatic traversal
     bool has_tree = false;             // built for the loaded scene
+    float boxes = 0.0f;                // TreeBuild::boxes: chooses the kernel of a pass
     uint32_t tree_walk = WALK_AUTO, tree_small_stack = 0;   // a test's (rsh_selfcheck_tree_walk)
     std::vector<float> host_light_pos;   // float4[L] as loaded
     // cluster level: CLUSTER consecutive triangles of one object per cluster
@@ -854,6 +855,7 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         q.obj_sphere = f4p(e->obj_sphere); q.obj_range = e->obj_range.as<uint4>();
         q.algorithm = cfg.algorithm; q.kind = kind; q.hit_mode = cfg.hit_mode;
         q.line_only = RSH_CAMERA_LINE_ONLY && camera && kind == 0 ? 1u : 0u;
+        q.boxes = e->boxes;
         q.walk = e->tree_walk; q.small_stack = e->tree_small_stack;
         q.closest = u64p(closest); q.shadow = u32p(closest);       // by kind
         StageTimer t(L, ST_PASS_TRAVERSE + (int)pass_idx, trav_timing);
@@ -1206,6 +1208,7 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
         HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
+    e->boxes = e->has_tree ? e->tree.boxes() : 0.0f;
     e->orig_ready = false;
     e->ranges_tb = 0xFFFFFFFFu;
     e->scene_epoch++;
@@ -2006,6 +2009,7 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
         HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
+    e->boxes = e->has_tree ? e->tree.boxes() : 0.0f;
     drop_graph(e);
     e->scene_epoch++;
     return RSH_OK;

@@ -14,6 +14,8 @@
 // children of the largest surface.  It is rebuilt on the device at scene load
 // and after object updates (262,604 triangles: 0.41 ms, bound by the
 // latency of its 26 launches and of the merging rounds).
+#include <cmath>
+#include <cstring>
 #include <utility>
 
 #include "rsh_kernels.hpp"
@@ -52,6 +54,11 @@ __device__ __forceinline__ float wave_max_f(float x) {
     return x;
 }
 
+__device__ __forceinline__ float half_surface(float4 lo, float4 hi) {
+    const float x = hi.x - lo.x, y = hi.y - lo.y, z = hi.z - lo.z;
+    return x * y + y * z + z * x;
+}
+
 // bounds: ordered words of the scene box (lo xyz, hi xyz) and the largest
 // triangle-sphere radius.
 __global__ void k_tree_clear(uint32_t* bounds) {
@@ -75,12 +82,13 @@ __global__ void k_tree_clear(uint32_t* bounds) {
 // a wave, 12 so).
 constexpr uint32_t PRIM_BLOCKS = 64;
 __global__ void __launch_bounds__(1024) k_tree_prims(const float4* tri_sphere, const float4* tri_mt, uint32_t T,
-                                                    float4* box, uint32_t* bounds) {
+                                                    float4* box, uint32_t* bounds, float* area) {
     __shared__ uint32_t s_bounds[7];
+    __shared__ float s_area[16];
     if (threadIdx.x < 7) s_bounds[threadIdx.x] = threadIdx.x < 3 ? ordered(INFINITY) : threadIdx.x < 6 ? ordered(-INFINITY) : ordered(0.0f);
     __syncthreads();
     v3 all_lo = mk(INFINITY, INFINITY, INFINITY), all_hi = mk(-INFINITY, -INFINITY, -INFINITY);
-    float all_r = 0.0f;
+    float all_r = 0.0f, sum = 0.0f;
     for (uint32_t t = blockIdx.x * 1024 + threadIdx.x; t < T; t += gridDim.x * 1024) {
         v3 lo = mk(INFINITY, INFINITY, INFINITY), hi = mk(-INFINITY, -INFINITY, -INFINITY);
         const v3 a = xyz(tri_mt[3 * (size_t)t]), e1 = xyz(tri_mt[3 * (size_t)t + 1]), e2 = xyz(tri_mt[3 * (size_t)t + 2]);
@@ -104,13 +112,17 @@ __global__ void __launch_bounds__(1024) k_tree_prims(const float4* tri_sphere, c
             all_lo = mk(fminf(all_lo.x, l.x), fminf(all_lo.y, l.y), fminf(all_lo.z, l.z));
             all_hi = mk(fmaxf(all_hi.x, h.x), fmaxf(all_hi.y, h.y), fmaxf(all_hi.z, h.z));
             all_r = fmaxf(all_r, s.w);
+            sum += half_surface(f4(l, 0.0f), f4(h, 0.0f));
         }
         box[2 * (size_t)t] = f4(lo, 0.0f);
         box[2 * (size_t)t + 1] = f4(hi, 0.0f);
     }
     const float m[7] = {wave_min_f(all_lo.x), wave_min_f(all_lo.y), wave_min_f(all_lo.z),
                         wave_max_f(all_hi.x), wave_max_f(all_hi.y), wave_max_f(all_hi.z), wave_max_f(all_r)};
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
     if ((threadIdx.x & 63u) == 0) {
+        s_area[threadIdx.x >> 6] = sum;
 #pragma unroll
         for (int i = 0; i < 3; i++) atomicMin(&s_bounds[i], ordered(m[i]));
 #pragma unroll
@@ -119,6 +131,11 @@ __global__ void __launch_bounds__(1024) k_tree_prims(const float4* tri_sphere, c
     __syncthreads();
     if (threadIdx.x < 3) atomicMin(&bounds[threadIdx.x], s_bounds[threadIdx.x]);
     else if (threadIdx.x < 7) atomicMax(&bounds[threadIdx.x], s_bounds[threadIdx.x]);
+    else if (threadIdx.x == 7) {
+        float all = 0.0f;
+        for (uint32_t i = 0; i < 16; i++) all += s_area[i];
+        area[blockIdx.x] = all;
+    }
 }
 
 __device__ __forceinline__ uint32_t spread10(uint32_t x) {
@@ -181,13 +198,11 @@ struct MergeArgs {
     uint32_t base;               // nodes of this launch: MERGE_CHUNK for each workgroup from here on
     float4* node;                // node i < T: i-th triangle in Morton order; (lo, left child), (hi, right child)
     uint32_t* size;              // triangles below a node >= T, and TREE_SPLIT
+    const float* area;           // half surfaces of the triangles' boxes, summed by each of area_blocks blocks
+    uint32_t area_blocks;
+    float* cost;                 // last launch: their sum over the root's
     bool last;
 };
-
-__device__ __forceinline__ float half_surface(float4 lo, float4 hi) {
-    const float x = hi.x - lo.x, y = hi.y - lo.y, z = hi.z - lo.z;
-    return x * y + y * z + z * x;
-}
 
 template <bool FIRST>
 __global__ void __launch_bounds__(1024) k_tree_merge(MergeArgs A) {
@@ -325,6 +340,12 @@ __global__ void __launch_bounds__(1024) k_tree_merge(MergeArgs A) {
     }
     for (uint32_t i = tid; i < n; i += 1024) A.out[(size_t)blockIdx.x * MERGE_KEEP + i] = s_id[i];
     if (tid == 0) A.out_count[blockIdx.x] = n;
+    if (A.last && tid < 64) {
+        float sum = tid < A.area_blocks ? A.area[tid] : 0.0f;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
+        if (tid == 0) *A.cost = sum / surface(0);
+    }
 }
 
 // Wide node w, built from a binary node: the child of the largest surface is
@@ -732,15 +753,33 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
 // The same for small passes, a wave per ray: each step takes up to 16 entries
 // off the ray's stack, one to a quad, so a ray that meets hundreds of boxes is a
 // chain of tens of steps instead of hundreds.  It visits boxes that a nearer hit
-// would have spared, on SIMDs that a small pass leaves idle.  Traversal alone, a
-// quad and a wave per ray, 1000 / 8000 / 32000 / 64000 rays: office camera rays 53 /
-// 126 / 131 / 176 us and 18 / 30 / 83 / 165, diffuse rays of the 100k-triangle soup
-// 704 / 905 / 913 / 1021 and 65 / 91 / 216 / 382, of the 2k-triangle room 31 / 38 /
-// 53 / 53 and 14 / 21 / 46 / 77.  The line lies where the last of these meet;
-// camera rays, whose neighbours walk together, meet at half of it (16000 in the
-// room: 26 and 33 us, 32000: 42 and 61).
+// would have spared, on SIMDs that a small pass leaves idle.
 constexpr uint32_t WAVE_STACK = 512, SMALL_WAVE_STACK = 16;
-constexpr uint32_t WAVE_RAYS = 32768, WAVE_CAMERA_RAYS = 16384;
+
+// Up to how many rays a wave each is the faster.  How long a quad's chain of
+// steps is decides, and that goes with the triangle boxes a line through the
+// scene meets (TreeBuild::boxes).  Whole queries, quad and wave in us:
+//   boxes  scene                  33000 rays    65536        131072
+//     6    plain room, diffuse     131   144   144   180    156   243
+//    13    atrium, diffuse         227   169   199   220    226   338
+//    25    office, primary         211   170   226   243    247   400
+//    25    office, diffuse         193   166   227   229    256   365
+//    29    soup of 10k, diffuse    448   220   490   300    568   489
+//   115    2k large triangles      878   257   911   395   1080   648
+//   170    100k, sparse            305   199   346   276    423   441
+//   259    soup of 100k, primary   672   257   730   506   1203   697
+//   259    soup of 100k, diffuse   982   313  1119   488   1363   845
+// The limit is 32768 up to 12 boxes, where the plain room's lie together, and
+// grows with them to four times that, where the first of the long ones meet.
+// With 32768 for all, 33,000 rays of the long scenes were slower than by testing
+// every candidate (soup, primary 579; 10k, diffuse 364; large triangles 428).
+// Camera rays, whose neighbours walk together, meet at half of it and at most at
+// three times that (49152 rays, quad and wave: office 297 and 326, soup 523 and
+// 509, 100k overlapping 498 and 489; 76800: soup 568 and 673).
+inline uint32_t wave_rays(const TreeParams& p) {
+    const float f = std::fmin(p.line_only ? 3.0f : 4.0f, std::fmax(1.0f, p.boxes / 12.0f));
+    return (uint32_t)((p.line_only ? 16384.0f : 32768.0f) * f);
+}
 
 template <int KIND, uint32_t CAP>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace_wave(const TreeParams P) {
@@ -896,12 +935,15 @@ hipError_t TreeBuild::reserve(uint32_t T) {
     size_t binary = 2 * (size_t)T;
     for (uint32_t g = groups; g > 1;) { g = (g + 15) / 16; binary += (size_t)g * MERGE_CHUNK; }
     const size_t wide = wide_nodes(T);
-    hipError_t e = hipSuccess;
+    hipError_t e = acquire_words(cost, 64,
+        [](void** p, size_t n) { return hipHostMalloc(p, n, hipHostMallocCoherent | hipHostMallocMapped); },
+        [](void** d, void* p) { return hipHostGetDevicePointer(d, p, 0); }, [](void* p) { return hipHostFree(p); });
     for (int pass = 0; pass < 2 && e == hipSuccess; pass++) {      // sizes, then addresses
         Slab a{pass ? keep.as<char>() : nullptr}, b{pass ? work.as<char>() : nullptr};
         a.take(nodes, wide * sizeof(TreeNode)); a.take(records, (size_t)T * 64); a.take(bounds, 64);
         b.take(box, (size_t)T * 32); b.take(node, binary * 32); b.take(size, binary * 4);
         b.take(left, ((size_t)groups * 2 + 2) * MERGE_KEEP * 4); b.take(left_count, ((size_t)groups * 2 + 2) * 4);
+        b.take(area, PRIM_BLOCKS * 4);
         b.take(scodes, (size_t)T * 4); b.take(sids, (size_t)T * 4); b.take(queue, wide * 8);
         b.take(count, (TREE_LEVELS + 1) * 4); b.take(codes, (size_t)T * 4); b.take(ids, (size_t)T * 4);
         b.take(sc.ping_k, (size_t)T * 4); b.take(sc.ping_v, (size_t)T * 4); b.take(sc.hist, sort_hist_bytes(T));
@@ -916,6 +958,14 @@ hipError_t TreeBuild::reserve(uint32_t T) {
 void TreeBuild::release() {
     keep.release();
     work.release();
+    if (cost.host) (void)hipHostFree(cost.host);
+    cost = HostWords{};
+}
+
+float TreeBuild::boxes() const {
+    float f = 0.0f;
+    if (cost.host) std::memcpy(&f, cost.host, 4);
+    return std::isfinite(f) ? f : 0.0f;
 }
 
 hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
@@ -924,7 +974,8 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
     float4* bx = box.as<float4>();
     uint32_t* bd = bounds.as<uint32_t>();
     k_tree_clear<<<1, 64, 0, s>>>(bd);
-    k_tree_prims<<<min(grid_for(T, 1024), PRIM_BLOCKS), 1024, 0, s>>>(tri_sphere, tri_mt, T, bx, bd);
+    const uint32_t prim_blocks = min(grid_for(T, 1024), PRIM_BLOCKS);
+    k_tree_prims<<<prim_blocks, 1024, 0, s>>>(tri_sphere, tri_mt, T, bx, bd, area.as<float>());
     k_tree_codes<<<grid_for(T, 256), 256, 0, s>>>(bx, T, bd, codes.as<uint32_t>(), ids.as<uint32_t>());
     const hipError_t e = run_radix_sort(codes.as<uint32_t>(), ids.as<uint32_t>(), T, 3 * CODE_BITS,
                                         scodes.as<uint32_t>(), sids.as<uint32_t>(), sc, s);
@@ -933,6 +984,7 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
     M.T = T; M.ids = sids.as<uint32_t>(); M.box = bx; M.base = T;
     M.node = node.as<float4>(); M.size = size.as<uint32_t>();
     M.out = left.as<uint32_t>(); M.out_count = left_count.as<uint32_t>();
+    M.area = area.as<float>(); M.area_blocks = prim_blocks; M.cost = reinterpret_cast<float*>(cost.dev);
     uint32_t groups = (T + MERGE_CHUNK - 1) / MERGE_CHUNK;
     M.last = groups == 1;
     k_tree_merge<true><<<groups, 1024, 0, s>>>(M);
@@ -965,8 +1017,7 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
 
 void launch_tree_trace(const TreeParams& p, hipStream_t s) {
     if (!p.N) return;
-    const bool small = p.N <= (p.line_only ? WAVE_CAMERA_RAYS : WAVE_RAYS);
-    const bool wave = !p.ps && (p.walk == WALK_WAVE || (p.walk != WALK_QUAD && small));
+    const bool wave = !p.ps && (p.walk == WALK_WAVE || (p.walk != WALK_QUAD && p.N <= wave_rays(p)));
     auto kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, WAVE_STACK> : k_tree_trace_wave<0, WAVE_STACK>)
                        : (p.kind == 1 ? k_tree_trace<1, STACK> : k_tree_trace<0, STACK>);
     if (p.small_stack)

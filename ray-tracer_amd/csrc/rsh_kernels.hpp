@@ -2,6 +2,7 @@
 // surface, shading, hierarchy and traversal stages.
 #pragma once
 #include "fastdiv.hpp"
+#include "host_words.hpp"
 #include "rsh_internal.hpp"
 
 namespace rsh {
@@ -335,10 +336,15 @@ constexpr uint32_t TREE_MAX_TRIANGLES = 1u << 29;      // places in a child word
 struct TreeBuild {
     DevBuf nodes, records, bounds;                                          // what the traversal reads (parts of keep)
     // construction (parts of work)
-    DevBuf box, node, size, left, left_count, codes, ids, scodes, sids, queue, count;
+    DevBuf box, node, size, left, left_count, area, codes, ids, scodes, sids, queue, count;
     ScanScratch sc;                                                         // the sort's scratch (part of work)
     DevBuf keep, work;
+    HostWords cost;                                                         // float, as boxes() returns it
     hipError_t reserve(uint32_t T);
+    // Once a build has ended on its stream: the surface of the triangles' boxes
+    // over that of the scene's, which is how many of them a line through the
+    // scene meets (0 where it is not finite).
+    float boxes() const;
     // objects: per object (first triangle, ...), K of them tiling [0, T) in order
     hipError_t build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
                      hipStream_t s);
@@ -364,6 +370,7 @@ struct TreeParams {
     const float4* obj_sphere;
     const uint4* obj_range;
     uint32_t algorithm, kind, hit_mode, line_only;
+    float boxes;                  // TreeBuild::boxes
     uint32_t walk, small_stack;   // a test's (rsh_selfcheck_tree_walk)
     unsigned long long* closest;  // kind 0: every traced ray's record is written
     uint32_t* shadow;             // kind 1: MISS32 where occluded

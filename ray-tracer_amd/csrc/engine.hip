@@ -679,7 +679,7 @@ rsh_status build_items(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, Trav
 rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const float* rays, uint32_t S,
                       uint32_t kind, const float4* shadow_pos, uint32_t flags_mask, PassOut& out, uint32_t pass_idx,
                       DevBuf& closest, const float* tmax = nullptr, bool camera = false, uint32_t sort_bits = 0,
-                      bool presorted = false, const float* front_point = nullptr) {
+                      bool presorted = false, const float* front_point = nullptr, bool query = false) {
     out = PassOut{};
     hipStream_t s = L.stream;
     const bool timing = flags_mask & 4u, counting = flags_mask & 2u;
@@ -855,7 +855,7 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         q.obj_sphere = f4p(e->obj_sphere); q.obj_range = e->obj_range.as<uint4>();
         q.algorithm = cfg.algorithm; q.kind = kind; q.hit_mode = cfg.hit_mode;
         q.line_only = RSH_CAMERA_LINE_ONLY && camera && kind == 0 ? 1u : 0u;
-        q.boxes = e->boxes;
+        q.boxes = e->boxes; q.frame = query ? 0u : 1u;
         q.walk = e->tree_walk; q.small_stack = e->tree_small_stack;
         q.closest = u64p(closest); q.shadow = u32p(closest);       // by kind
         StageTimer t(L, ST_PASS_TRAVERSE + (int)pass_idx, trav_timing);
@@ -1798,7 +1798,8 @@ rsh_status rsh_engine_trace(rsh_engine* e, const float* rays, const float* tmax,
         HIP_OK(hipGetLastError());
     }
     PassOut po;
-    if ((rs = trace_pass(e, L, cfg, rays, n, kind, nullptr, fl, po, 0, e->closest[0], tmax)) != RSH_OK) {
+    if ((rs = trace_pass(e, L, cfg, rays, n, kind, nullptr, fl, po, 0, e->closest[0], tmax, false, 0, false, nullptr,
+                         true)) != RSH_OK) {
         e->err = L.err;
         return rs;
     }

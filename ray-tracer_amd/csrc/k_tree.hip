@@ -14,6 +14,7 @@
 // children of the largest surface.  It is rebuilt on the device at scene load
 // and after object updates (262,604 triangles: 0.41 ms, bound by the
 // latency of its 26 launches and of the merging rounds).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -773,12 +774,17 @@ constexpr uint32_t WAVE_STACK = 512, SMALL_WAVE_STACK = 16;
 // grows with them to four times that, where the first of the long ones meet.
 // With 32768 for all, 33,000 rays of the long scenes were slower than by testing
 // every candidate (soup, primary 579; 10k, diffuse 364; large triangles 428).
-// Camera rays, whose neighbours walk together, meet at half of it and at most at
-// three times that (49152 rays, quad and wave: office 297 and 326, soup 523 and
-// 509, 100k overlapping 498 and 489; 76800: soup 568 and 673).
+// A frame's rays walk together, and a quad's chains are the shorter for it:
+// camera and mirror rays meet at half as many (office frame of 512x512, 44,000
+// mirror rays: 483 us with a quad a ray, 510 with a wave), camera rays at 49152 at
+// most (quad and wave: office 297 and 326, soup 523 and 509, 100k overlapping 498
+// and 489; 76800: soup 568 and 673), and shadow rays, which end at the first
+// occluder, not above 32768 in any scene (soup, 512x512, 90,000: 853 and 963).
 inline uint32_t wave_rays(const TreeParams& p) {
-    const float f = std::fmin(p.line_only ? 3.0f : 4.0f, std::fmax(1.0f, p.boxes / 12.0f));
-    return (uint32_t)((p.line_only ? 16384.0f : 32768.0f) * f);
+    const uint32_t rays = (uint32_t)(32768.0f * std::fmin(8.0f, std::fmax(1.0f, p.boxes / 12.0f)));     // of a query, unbounded
+    if (!p.frame) return std::min(rays, 131072u);
+    if (p.kind == 1) return 32768u;
+    return p.line_only ? std::min(rays / 2, 49152u) : std::min(std::max(rays / 2, 32768u), 131072u);
 }
 
 template <int KIND, uint32_t CAP>

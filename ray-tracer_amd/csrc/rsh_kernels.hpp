@@ -371,6 +371,7 @@ struct TreeParams {
     const uint4* obj_range;
     uint32_t algorithm, kind, hit_mode, line_only;
     float boxes;                  // TreeBuild::boxes
+    uint32_t frame;               // a frame's pass (0: a query's)
     uint32_t walk, small_stack;   // a test's (rsh_selfcheck_tree_walk)
     unsigned long long* closest;  // kind 0: every traced ray's record is written
     uint32_t* shadow;             // kind 1: MISS32 where occluded

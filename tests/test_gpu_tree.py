@@ -405,3 +405,26 @@ def test_overlapping_scenes_are_no_slower_than_without_the_tree(engine, rsh, wal
     tree = query_ms(engine, rsh, rays, cfg)
     walk(NO_TREE)
     assert tree < query_ms(engine, rsh, rays, cfg)
+
+
+def frame_ms(engine, cam, cfg, flags):
+    import time
+    times = []
+    for _ in range(20):
+        t = time.perf_counter()
+        engine.render(cam, cfg, flags=flags)
+        times.append(time.perf_counter() - t)
+    return 1e3 * min(times)
+
+
+def test_a_frames_shadow_rays_keep_a_quad_each(engine, rsh, walk):
+    """90,000 of them in a 512x512 frame of the soup: they end at the first
+    occluder, so a wave each is the slower by 13 % of the frame."""
+    sc = rsh.scenes.soup_scene()
+    engine.load_scene(sc)
+    cfg = dataclasses.replace(rsh.config.config0(512, 512), bounces=0, bounce_shadows=0).with_scene_bounds(sc)
+    cam = rsh.scenes.random_view(np.random.default_rng(1), 512, 512)
+    auto = frame_ms(engine, cam, cfg, 0)
+    assert 60_000 < engine.stats.pass_rays[1] < 131_072
+    walk(QUAD)
+    assert auto < 1.06 * frame_ms(engine, cam, cfg, 0)

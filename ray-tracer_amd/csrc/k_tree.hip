@@ -780,8 +780,11 @@ constexpr uint32_t WAVE_STACK = 512, SMALL_WAVE_STACK = 16;
 // most (quad and wave: office 297 and 326, soup 523 and 509, 100k overlapping 498
 // and 489; 76800: soup 568 and 673), and shadow rays, which end at the first
 // occluder, not above 32768 in any scene (soup, 512x512, 90,000: 853 and 963).
+// A device-sized pass, as captured frames have, is taken by its capacity: the
+// workgroups past its rays end at once (replayed 64x64 frame with two bounces
+// and shadows, soup: 1275 us with a quad a ray, 438 so).
 inline uint32_t wave_rays(const TreeParams& p) {
-    const uint32_t rays = (uint32_t)(32768.0f * std::fmin(8.0f, std::fmax(1.0f, p.boxes / 12.0f)));     // of a query, unbounded
+    const uint32_t rays = (uint32_t)(32768.0f * std::fmin(8.0f, std::fmax(1.0f, p.boxes / 12.0f)));     // a query's, before its cap
     if (!p.frame) return std::min(rays, 131072u);
     if (p.kind == 1) return 32768u;
     return p.line_only ? std::min(rays / 2, 49152u) : std::min(std::max(rays / 2, 32768u), 131072u);
@@ -792,8 +795,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
     __shared__ uint32_t s_stack[CAP];
     __shared__ uint16_t s_near[KIND == 0 ? CAP : 1];    // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, quad = lane >> 2, pos = blockIdx.x;
-    if (pos >= P.N) return;
-    const uint32_t* off = P.level_offset;
+    if (pos >= (P.ps ? P.ps->N : P.N)) return;
+    const uint32_t* off = P.ps ? P.ps->offset : P.level_offset;
     const float4 r0 = P.rec0[pos], r1 = P.rec1[pos];
     const v3 d = xyz(r1), o = xyz(r0) + d * EPS;
     const float dd = dot(d, d);
@@ -1023,7 +1026,7 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
 
 void launch_tree_trace(const TreeParams& p, hipStream_t s) {
     if (!p.N) return;
-    const bool wave = !p.ps && (p.walk == WALK_WAVE || (p.walk != WALK_QUAD && p.N <= wave_rays(p)));
+    const bool wave = p.walk == WALK_WAVE || (p.walk != WALK_QUAD && p.N <= wave_rays(p));
     auto kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, WAVE_STACK> : k_tree_trace_wave<0, WAVE_STACK>)
                        : (p.kind == 1 ? k_tree_trace<1, STACK> : k_tree_trace<0, STACK>);
     if (p.small_stack)

@@ -524,7 +524,7 @@ __global__ void __launch_bounds__(256) k_tree_records(EmitArgs A, const uint32_t
 // (k_traverse64) with its culling and work list, traversal alone: the frame's
 // 8 passes 4.77 -> 1.84 ms, a query of 1M diffuse rays 9.18 -> 0.52 ms, one of
 // 100k shadow rays 0.54 -> 0.12 ms.
-constexpr uint32_t STACK = 48, SMALL_STACK = 6;       // the latter for the tests of a full stack
+constexpr uint32_t STACK = 48, SMALL_STACK = 6;       // the latter: used of it in the tests of a full stack
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t quad_u(uint32_t x) {
@@ -580,7 +580,7 @@ __device__ __forceinline__ Slabs make_slabs(const TreeParams& P, v3 o, v3 d, flo
                        fmaxf(fabsf(slo.z - o.z), fabsf(shi.z - o.z));
     const float e = 1.1e-4f * (far1 + unordered(P.bounds[6])) + 1e-5f;
     const v3 ao = mk(fabsf(o.x), fabsf(o.y), fabsf(o.z));
-    const v3 m = mk(e + 4e-7f * ao.x, e + 4e-7f * ao.y, e + 4e-7f * ao.z);
+    const v3 m = mk(__builtin_fmaf(4e-7f, ao.x, e), __builtin_fmaf(4e-7f, ao.y, e), __builtin_fmaf(4e-7f, ao.z, e));
     // Rays whose magnitudes leave the range of the slab arithmetic visit every
     // box (all factors 0: no box is rejected).
     s.plain = dd >= 1e-24f && dd <= 1e24f && far1 + fmaxf(ao.x, fmaxf(ao.y, ao.z)) <= 1e15f;
@@ -605,10 +605,10 @@ __device__ __forceinline__ bool meets(const Slabs& s, float4 lo, float4 hi, floa
     return !(tn > tf) && __float_as_uint(lo.w) != TREE_EMPTY;
 }
 
-template <int KIND, uint32_t CAP>
+template <int KIND>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace(const TreeParams P) {
-    __shared__ uint32_t s_stack[CAP][16];
-    __shared__ uint16_t s_near[KIND == 0 ? CAP : 1][16];     // entry distance, upper half (rounded down)
+    __shared__ uint32_t s_stack[STACK][16];
+    __shared__ uint16_t s_near[KIND == 0 ? STACK : 1][16];     // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, ray = lane >> 2;
     const uint32_t* off = P.ps ? P.ps->offset : P.level_offset;
     // Workgroups go to the 8 XCDs in turn; 64 neighbours (1024 sorted rays) stay
@@ -658,7 +658,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
             // rank of the lane's child among the hit ones, nearest first
             const uint32_t rank = (quad_u<QUAD_ROT1>(key) < key ? 1u : 0u) + (quad_u<QUAD_ROT2>(key) < key ? 1u : 0u) +
                                   (quad_u<QUAD_ROT3>(key) < key ? 1u : 0u);
-            const bool full = sp + n > CAP;    // no ray of a scene of ordinary depth
+            const bool full = sp + n > P.stack;    // no ray of a scene of ordinary depth
             if (in && !full) {
                 const uint32_t at = sp + n - 1u - rank;
                 s_stack[at][ray] = ch;
@@ -790,10 +790,10 @@ inline uint32_t wave_rays(const TreeParams& p) {
     return p.line_only ? std::min(rays / 2, 49152u) : std::min(std::max(rays / 2, 32768u), 131072u);
 }
 
-template <int KIND, uint32_t CAP>
+template <int KIND>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8))) k_tree_trace_wave(const TreeParams P) {
-    __shared__ uint32_t s_stack[CAP];
-    __shared__ uint16_t s_near[KIND == 0 ? CAP : 1];    // entry distance, upper half (rounded down)
+    __shared__ uint32_t s_stack[WAVE_STACK];
+    __shared__ uint16_t s_near[KIND == 0 ? WAVE_STACK : 1];    // entry distance, upper half (rounded down)
     const uint32_t lane = threadIdx.x, q = lane & 3u, quad = lane >> 2, pos = blockIdx.x;
     if (pos >= (P.ps ? P.ps->N : P.N)) return;
     const uint32_t* off = P.ps ? P.ps->offset : P.level_offset;
@@ -819,7 +819,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8, 8)))
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");     // pushed by one lane, taken by others
         uint32_t j = TREE_EMPTY;               // the lane's triangle
         if (sp != 0u) {
-            const uint32_t m = min(min(sp, 16u), (CAP - sp) / 3u);
+            const uint32_t m = min(min(sp, 16u), (P.stack - sp) / 3u);
             if (m == 0u) {                     // full: the ray takes every triangle in turn
                 sp = 0u;
                 scan = 0u;
@@ -1027,12 +1027,16 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
 void launch_tree_trace(const TreeParams& p, hipStream_t s) {
     if (!p.N) return;
     const bool wave = p.walk == WALK_WAVE || (p.walk != WALK_QUAD && p.N <= wave_rays(p));
-    auto kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, WAVE_STACK> : k_tree_trace_wave<0, WAVE_STACK>)
-                       : (p.kind == 1 ? k_tree_trace<1, STACK> : k_tree_trace<0, STACK>);
-    if (p.small_stack)
-        kernel = wave ? (p.kind == 1 ? k_tree_trace_wave<1, SMALL_WAVE_STACK> : k_tree_trace_wave<0, SMALL_WAVE_STACK>)
-                      : (p.kind == 1 ? k_tree_trace<1, SMALL_STACK> : k_tree_trace<0, SMALL_STACK>);
-    kernel<<<wave ? p.N : grid_for(p.N, 16), 64, 0, s>>>(p);
+    TreeParams q = p;
+    if (wave) {
+        q.stack = p.small_stack ? SMALL_WAVE_STACK : WAVE_STACK;
+        if (p.kind == 1) k_tree_trace_wave<1><<<p.N, 64, 0, s>>>(q);
+        else k_tree_trace_wave<0><<<p.N, 64, 0, s>>>(q);
+        return;
+    }
+    q.stack = p.small_stack ? SMALL_STACK : STACK;
+    if (p.kind == 1) k_tree_trace<1><<<grid_for(p.N, 16), 64, 0, s>>>(q);
+    else k_tree_trace<0><<<grid_for(p.N, 16), 64, 0, s>>>(q);
 }
 
 }  // namespace rsh

@@ -373,6 +373,7 @@ struct TreeParams {
     float boxes;                  // TreeBuild::boxes
     uint32_t frame;               // a frame's pass (0: a query's)
     uint32_t walk, small_stack;   // a test's (rsh_selfcheck_tree_walk)
+    uint32_t stack;               // entries of a ray's stack to use (set by the launch)
     unsigned long long* closest;  // kind 0: every traced ray's record is written
     uint32_t* shadow;             // kind 1: MISS32 where occluded
 };

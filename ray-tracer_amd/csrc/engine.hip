@@ -1128,7 +1128,10 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
         e->old_M = e->M;
         e->records_old = true;
     }
-    e->T = T; e->K = K; e->M = M; e->L = L;
+    // no scene until all of this one is there: a load that fails half-way leaves
+    // arrays of two scenes
+    e->T = 0;
+    e->K = K; e->M = M; e->L = L;
     HIP_OK(e->tri_pos.reserve((size_t)T * 48)); HIP_OK(e->tri_nrm.reserve((size_t)T * 48));
     HIP_OK(e->tri_mat.reserve((size_t)T * 12));
     HIP_OK(e->mat_dif.reserve((size_t)M * 16)); HIP_OK(e->mat_spec.reserve((size_t)M * 16));
@@ -1208,6 +1211,7 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
         HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));
+    e->T = T;
     e->boxes = e->has_tree ? e->tree.boxes() : 0.0f;
     e->orig_ready = false;
     e->ranges_tb = 0xFFFFFFFFu;

@@ -89,7 +89,9 @@ typedef struct rsh_frame_config {
     uint32_t traversal_kernel;      /* 0 automatic, 1 generic kernel for every shape.  The
                                        automatic traversal walks a tree over the scene's
                                        triangles unless one of the three fields below or
-                                       counters (flag bit 1) are asked for                */
+                                       counters (flag bit 1) are asked for; large camera
+                                       passes of scenes whose triangles overlap take the
+                                       64-ray kernel                                      */
     uint32_t traversal_splits;      /* generic kernel: waves per top node; 0 = fill the GPU */
     uint32_t traversal_chunk;       /* 64-ray kernel: candidate clusters (64 consecutive
                                        triangles of one object) per work item; 0 = sized

@@ -133,7 +133,13 @@ struct rsh_engine {
     DevBuf tri_sphere, tri_mt, obj_sphere, obj_range;
     TreeBuild tree;                    // triangle tree of the automatic traversal
     bool has_tree = false;             // built for the loaded scene
-    float boxes = 0.0f;                // TreeBuild::boxes: chooses the kernel of a pass
+    // what the tree's build wrote, in page-locked words behind lane 0's ord_host,
+    // and their device address
+    const TreeMeasure* measure = nullptr;
+    TreeMeasure* measure_dev = nullptr;
+    // What chooses a pass's kernel: TreeMeasure::boxes, and how many triangles a line
+    // through the scene meets when each object's sphere stands for all of its own
+    float boxes = 0.0f, covered = 0.0f;
     uint32_t tree_walk = WALK_AUTO, tree_small_stack = 0;   // a test's (rsh_selfcheck_tree_walk)
     std::vector<float> host_light_pos;   // float4[L] as loaded
     // cluster level: CLUSTER consecutive triangles of one object per cluster
@@ -169,6 +175,7 @@ struct rsh_engine {
     // replay (hrec); an overflow re-renders the frame eagerly.
     bool dev_sized = false;            // set while such a frame is captured
     bool gdev = false;                 // the current graph is device-sized
+    bool fronted = false, gfront = false;      // a pass of the frame, of the graph, ran front to back
     DevBuf frame_rec;                  // uint32[2 * RSH_MAX_PASSES + 1]: (N, C) per pass, overflow
     uint32_t* hrec = nullptr;          // page-locked copy of frame_rec
     hipGraph_t graph = nullptr;
@@ -510,6 +517,29 @@ void build_clusters(rsh_engine* e, hipStream_t st) {
     launch_sub_use(f4p(e->cl_sphere), f4p(e->sub_sphere), e->NC, e->sub_use.as<uint8_t>(), st);
 }
 
+// Sum over the objects of their sphere's squared radius times their triangles.
+// scale: the object updates' matrices (a radius times the largest diagonal entry).
+double object_spread(const rsh_engine* e, const float* scale) {
+    double sum = 0.0;
+    for (uint32_t k = 0; k < e->K; k++) {
+        const float* h = &e->host_spheres[6 * (size_t)k];
+        const float* m = scale ? scale + 16 * (size_t)k : nullptr;
+        const double r = m ? (double)h[3] * std::max(std::fabs(m[0]), std::max(std::fabs(m[5]), std::fabs(m[10]))) : h[3];
+        sum += r * r * ((double)h[5] - h[4] + 1.0);
+    }
+    return sum;
+}
+
+// What chooses a pass's kernel, once the tree's build has ended.
+void measure_scene(rsh_engine* e, double spread) {
+    const bool ok = e->has_tree && std::isfinite(e->measure->boxes) && std::isfinite(e->measure->half_root);
+    const float root = ok ? e->measure->half_root : 0.0f;
+    e->boxes = root > 0.0f ? e->measure->boxes : 0.0f;
+    // a line through the scene meets a sphere in it by its surface over the scene's
+    const double covered = root > 0.0f ? 2.0 * 3.14159265 * spread / root : 0.0;
+    e->covered = covered <= (double)e->T ? (float)covered : (float)e->T;
+}
+
 struct PassOut {
     uint32_t N = 0, C = 0, splits = 0, items = 0, chunk = 0;
     uint64_t top = 0, leaf = 0, tests = 0, surv = 0, tri_tests = 0, cl_tests = 0, b_steps = 0, c_steps = 0;
@@ -671,6 +701,55 @@ rsh_status build_items(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, Trav
         pp.chunk = chunk; pp.list_total = tot[0]; pp.items = tot[1]; pp.mode = p.prefilter;
     }
     return RSH_OK;
+}
+
+// The objects by the distance from the point to their spheres as loaded (moved
+// objects keep their loaded place: the order only steers the pruning, never a
+// result), into the lane's page-locked words.
+void front_order(rsh_engine* e, Lane& L, const float* point) {
+    std::vector<std::pair<float, uint32_t>> dk(e->K);
+    for (uint32_t k = 0; k < e->K; k++) {
+        const float* h = &e->host_spheres[6 * (size_t)k];
+        const float dx = h[0] - point[0], dy = h[1] - point[1], dz = h[2] - point[2];
+        const float d = std::sqrt(dx * dx + dy * dy + dz * dz) - h[3];
+        dk[k] = {d > 0.0f ? d : 0.0f, k};
+    }
+    std::sort(dk.begin(), dk.end());
+    for (uint32_t k = 0; k < e->K; k++) L.ord_host[k] = dk[k].second;
+}
+
+// The 64-ray kernel's shapes.
+bool items_shape(const rsh_frame_config& c) {
+    return c.depth == 2 && c.leaf * c.branch == 64 && c.traversal_kernel != 1 &&
+           (c.leaf == 2 || c.leaf == 4 || c.leaf == 8 || c.leaf == 16 || c.leaf == 32);
+}
+
+// Large camera passes of scenes whose triangles overlap within objects apart from
+// one another: 64 neighbouring rays share one list of candidates there, while in
+// the tree each meets all the boxes by itself.  Frames without bounces, the camera
+// pass in the tree and by candidates in us, by the boxes and the covered triangles
+// that a line meets:
+//   boxes covered  scene                 196608       262144        2073600
+//     6     110    plain room           260  422     284  447      687   979
+//    25      58    office              373  613     367  634     1174  2006
+//    29     163    soup of 10k          667  720     669  726     2125  1815
+//    81     478    soup of 30k          611  619     698  744     2961  1886
+//   115    1084    2k large triangles   779  512     871  557     3904  2151
+//   132     616    50k, 1001 objects    589  753     661  835     2411  2422
+//   259    1565    soup of 100k         863  781    1033  799     5643  2985
+//   338   11026    20k, wide objects   1095 1486    1266 1725     6077 10761
+//   801    7510    20k large           3206 1576    3603 2001    17919 13822
+//  1022    6229    soup of 400k        1752 1016    2023 1202    11284  5520
+// From these about 0.3 + 0.02 boxes ns a ray in the tree, 0.45 + 0.0002 objects +
+// 0.0008 covered by candidates and, for their lists, 250 us + 0.4 an object.  The
+// candidates have to look a quarter faster (balls of 128 triangles, 52 boxes and
+// 768 covered: 971 in the tree, 1365 by candidates), and below 196608 rays the
+// soup's lie the other way round (131072: 664 and 900).  Only for a single view
+// and exact hits, whose objects are taken front to back.
+bool by_candidates(const rsh_engine* e, const rsh_frame_config& cfg, uint32_t N) {
+    if (N < 196608u || cfg.algorithm != RSH_CRSH || cfg.hit_mode != 0 || !items_shape(cfg)) return false;
+    const float K = (float)e->K, tree = 0.3f + 0.02f * e->boxes, cand = 0.45f + 2e-4f * K + 8e-4f * e->covered;
+    return cand < 0.75f * tree && (float)N * (tree - cand) >= 2.5e5f + 400.0f * K;
 }
 
 // One ray batch: trim -> (compress -> sort -> decompress) -> gather ->
@@ -843,7 +922,9 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
     // The automatic traversal walks the triangle tree; a caller that counts
     // the reference's tests or picks a kernel, a work split or a pre-test gets
     // the kernels these belong to.
-    if (e->has_tree && e->tree_walk != WALK_NONE && !counting && cfg.traversal_kernel == 0 &&
+    const bool cands = e->tree_walk == WALK_NONE ||
+                       (e->tree_walk == WALK_AUTO && kind == 0 && camera && front_point && by_candidates(e, cfg, N));
+    if (e->has_tree && !cands && !counting && cfg.traversal_kernel == 0 &&
         cfg.traversal_prefilter == 0 && cfg.traversal_chunk == 0 && cfg.traversal_splits == 0) {
         TreeParams q{};
         q.tree = e->tree.nodes.as<TreeNode>(); q.records = f4p(e->tree.records); q.bounds = u32p(e->tree.bounds);
@@ -904,18 +985,8 @@ rsh_status trace_pass(rsh_engine* e, Lane& L, const rsh_frame_config& cfg, const
         // cull + work list; its time (host read-backs included) counts as traversal
         StageTimer t(L, ST_TRAVERSE, timing);
         if (front) {
-            // by the distance from the point to each object's sphere as loaded
-            // (moved objects keep their loaded place: the order only steers
-            // the pruning, never a result)
-            std::vector<std::pair<float, uint32_t>> dk(e->K);
-            for (uint32_t k = 0; k < e->K; k++) {
-                const float* h = &e->host_spheres[6 * (size_t)k];
-                const float dx = h[0] - front_point[0], dy = h[1] - front_point[1], dz = h[2] - front_point[2];
-                const float d = std::sqrt(dx * dx + dy * dy + dz * dz) - h[3];
-                dk[k] = {d > 0.0f ? d : 0.0f, k};
-            }
-            std::sort(dk.begin(), dk.end());
-            for (uint32_t k = 0; k < e->K; k++) L.ord_host[k] = dk[k].second;
+            front_order(e, L, front_point);
+            e->fronted = true;
             LANE_OK(hipMemcpyAsync(L.obj_order.p, L.ord_host, (size_t)e->K * 4, hipMemcpyHostToDevice, s));
             p.obj_order = u32p(L.obj_order);
         }
@@ -1129,7 +1200,7 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
         e->records_old = true;
     }
     // no scene until all of this one is there: a load that fails half-way leaves
-    // arrays of two scenes
+    // arrays of two scenes, and page-locked words that are freed
     e->T = 0;
     e->K = K; e->M = M; e->L = L;
     HIP_OK(e->tri_pos.reserve((size_t)T * 48)); HIP_OK(e->tri_nrm.reserve((size_t)T * 48));
@@ -1142,8 +1213,13 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     for (Lane& l : e->lane) {
         HIP_OK(l.obj_order.reserve((size_t)K * 4 + 4));
         if (l.ord_host) { (void)hipHostFree(l.ord_host); l.ord_host = nullptr; }
-        HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&l.ord_host), (size_t)K * 4 + 4, hipHostMallocDefault));
+        HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&l.ord_host), (size_t)K * 4 + 4 + sizeof(TreeMeasure),
+                             hipHostMallocDefault));
     }
+    e->measure = reinterpret_cast<const TreeMeasure*>(e->lane[0].ord_host + K);
+    void* words = nullptr;
+    HIP_OK(hipHostGetDevicePointer(&words, e->lane[0].ord_host, 0));
+    e->measure_dev = reinterpret_cast<TreeMeasure*>(static_cast<uint32_t*>(words) + K);
     hipStream_t st = e->stream;
     HIP_OK(hipMemcpyAsync(e->tri_pos.p, s->tri_pos, (size_t)T * 48, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(e->tri_nrm.p, s->tri_nrm, (size_t)T * 48, hipMemcpyHostToDevice, st));
@@ -1208,11 +1284,12 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
         }
     }
     if (e->has_tree)
-        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
+        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, e->measure_dev, st));
     HIP_OK(hipGetLastError());
+    const double spread = object_spread(e, nullptr);
     HIP_OK(hipStreamSynchronize(st));
     e->T = T;
-    e->boxes = e->has_tree ? e->tree.boxes() : 0.0f;
+    measure_scene(e, spread);
     e->orig_ready = false;
     e->ranges_tb = 0xFFFFFFFFu;
     e->scene_epoch++;
@@ -1584,9 +1661,7 @@ void drop_graph(rsh_engine* e) {
 // Shadow and reflection passes of this configuration can keep their sizes on
 // the device: CRSH with the 64-ray traversal kernel, single-block item scans.
 bool dev_sizable(const rsh_engine* e, const rsh_frame_config& cfg, uint64_t slots) {
-    if (cfg.algorithm != RSH_CRSH || cfg.depth != 2 || cfg.leaf * cfg.branch != 64 || cfg.traversal_kernel == 1)
-        return false;
-    if (cfg.leaf != 2 && cfg.leaf != 4 && cfg.leaf != 8 && cfg.leaf != 16 && cfg.leaf != 32) return false;
+    if (cfg.algorithm != RSH_CRSH || !items_shape(cfg)) return false;
     const uint64_t n0 = (slots + cfg.leaf - 1) / cfg.leaf, ntop = (n0 + cfg.branch - 1) / cfg.branch;
     return ntop + 1 <= SMALL_SCAN && e->K > 0;
 }
@@ -1643,6 +1718,9 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
         e->records_old = false;
         if (e->gdev)
             HIP_OK(hipMemcpyAsync(e->views_d.p, hv, (size_t)nv * sizeof(ViewDesc), hipMemcpyHostToDevice, e->stream));
+        // the graph copies the order from these words: this camera's, not the
+        // captured one's (soup of 400k, another camera: 11.4 -> 4.6 ms)
+        if (e->gdev && e->gfront) front_order(e, e->lane[0], hv[0].eye);
         HIP_OK(hipGraphLaunch(e->gexec, e->stream));
         if (e->gdev)
             HIP_OK(hipMemcpyAsync(e->hrec, e->frame_rec.p, (2 * RSH_MAX_PASSES + 1) * 4, hipMemcpyDeviceToHost,
@@ -1706,6 +1784,7 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
     e->replaying = true;
     e->dev_sized = use_dev;
     for (Lane& l : e->lane) l.plan_pos = 0;
+    e->fronted = false;
     HIP_OK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeRelaxed));
     rs = render_frame(e, hv, nv, cfg, 0, nullptr);
     hipGraph_t g = nullptr;
@@ -1723,6 +1802,7 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
     const hipError_t ie = hipGraphInstantiate(&e->gexec, g, nullptr, nullptr, 0);
     if (ie != hipSuccess) { (void)hipGraphDestroy(g); e->gexec = nullptr; HIP_OK(ie); }
     e->graph = g; e->gsig = signature(!use_dev); e->gepoch = epoch; e->gstats = local; e->gdev = use_dev;
+    e->gfront = e->fronted;
     return RSH_OK;
 }
 
@@ -2011,10 +2091,11 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
     launch_triangle_prep(f4p(e->tri_pos), T, f4p(e->tri_sphere), f4p(e->tri_mt), st);
     build_clusters(e, st);
     if (e->has_tree)
-        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, st));
+        HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, e->measure_dev, st));
     HIP_OK(hipGetLastError());
+    const double spread = object_spread(e, scale);
     HIP_OK(hipStreamSynchronize(st));
-    e->boxes = e->has_tree ? e->tree.boxes() : 0.0f;
+    measure_scene(e, spread);
     drop_graph(e);
     e->scene_epoch++;
     return RSH_OK;

@@ -16,7 +16,6 @@
 // latency of its 26 launches and of the merging rounds).
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 #include <utility>
 
 #include "rsh_kernels.hpp"
@@ -201,7 +200,7 @@ struct MergeArgs {
     uint32_t* size;              // triangles below a node >= T, and TREE_SPLIT
     const float* area;           // half surfaces of the triangles' boxes, summed by each of area_blocks blocks
     uint32_t area_blocks;
-    float* cost;                 // last launch: their sum over the root's
+    TreeMeasure* measure;        // written by the last launch
     bool last;
 };
 
@@ -345,7 +344,10 @@ __global__ void __launch_bounds__(1024) k_tree_merge(MergeArgs A) {
         float sum = tid < A.area_blocks ? A.area[tid] : 0.0f;
 #pragma unroll
         for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, 64);
-        if (tid == 0) *A.cost = sum / surface(0);
+        if (tid == 0) {
+            const float root = surface(0);
+            *A.measure = TreeMeasure{sum / root, root};
+        }
     }
 }
 
@@ -759,7 +761,7 @@ constexpr uint32_t WAVE_STACK = 512, SMALL_WAVE_STACK = 16;
 
 // Up to how many rays a wave each is the faster.  How long a quad's chain of
 // steps is decides, and that goes with the triangle boxes a line through the
-// scene meets (TreeBuild::boxes).  Whole queries, quad and wave in us:
+// scene meets (TreeMeasure::boxes).  Whole queries, quad and wave in us:
 //   boxes  scene                  33000 rays    65536        131072
 //     6    plain room, diffuse     131   144   144   180    156   243
 //    13    atrium, diffuse         227   169   199   220    226   338
@@ -944,15 +946,12 @@ hipError_t TreeBuild::reserve(uint32_t T) {
     size_t binary = 2 * (size_t)T;
     for (uint32_t g = groups; g > 1;) { g = (g + 15) / 16; binary += (size_t)g * MERGE_CHUNK; }
     const size_t wide = wide_nodes(T);
-    hipError_t e = acquire_words(cost, 64,
-        [](void** p, size_t n) { return hipHostMalloc(p, n, hipHostMallocCoherent | hipHostMallocMapped); },
-        [](void** d, void* p) { return hipHostGetDevicePointer(d, p, 0); }, [](void* p) { return hipHostFree(p); });
+    hipError_t e = hipSuccess;
     for (int pass = 0; pass < 2 && e == hipSuccess; pass++) {      // sizes, then addresses
         Slab a{pass ? keep.as<char>() : nullptr}, b{pass ? work.as<char>() : nullptr};
         a.take(nodes, wide * sizeof(TreeNode)); a.take(records, (size_t)T * 64); a.take(bounds, 64);
         b.take(box, (size_t)T * 32); b.take(node, binary * 32); b.take(size, binary * 4);
         b.take(left, ((size_t)groups * 2 + 2) * MERGE_KEEP * 4); b.take(left_count, ((size_t)groups * 2 + 2) * 4);
-        b.take(area, PRIM_BLOCKS * 4);
         b.take(scodes, (size_t)T * 4); b.take(sids, (size_t)T * 4); b.take(queue, wide * 8);
         b.take(count, (TREE_LEVELS + 1) * 4); b.take(codes, (size_t)T * 4); b.take(ids, (size_t)T * 4);
         b.take(sc.ping_k, (size_t)T * 4); b.take(sc.ping_v, (size_t)T * 4); b.take(sc.hist, sort_hist_bytes(T));
@@ -967,24 +966,17 @@ hipError_t TreeBuild::reserve(uint32_t T) {
 void TreeBuild::release() {
     keep.release();
     work.release();
-    if (cost.host) (void)hipHostFree(cost.host);
-    cost = HostWords{};
-}
-
-float TreeBuild::boxes() const {
-    float f = 0.0f;
-    if (cost.host) std::memcpy(&f, cost.host, 4);
-    return std::isfinite(f) ? f : 0.0f;
 }
 
 hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
-                            hipStream_t s) {
+                            TreeMeasure* measure, hipStream_t s) {
     if (T == 0 || T > TREE_MAX_TRIANGLES || K == 0) return hipErrorInvalidValue;
     float4* bx = box.as<float4>();
     uint32_t* bd = bounds.as<uint32_t>();
     k_tree_clear<<<1, 64, 0, s>>>(bd);
     const uint32_t prim_blocks = min(grid_for(T, 1024), PRIM_BLOCKS);
-    k_tree_prims<<<prim_blocks, 1024, 0, s>>>(tri_sphere, tri_mt, T, bx, bd, area.as<float>());
+    float* sums = queue.as<float>();        // (256 B at least; the queue is filled after the merge has read them)
+    k_tree_prims<<<prim_blocks, 1024, 0, s>>>(tri_sphere, tri_mt, T, bx, bd, sums);
     k_tree_codes<<<grid_for(T, 256), 256, 0, s>>>(bx, T, bd, codes.as<uint32_t>(), ids.as<uint32_t>());
     const hipError_t e = run_radix_sort(codes.as<uint32_t>(), ids.as<uint32_t>(), T, 3 * CODE_BITS,
                                         scodes.as<uint32_t>(), sids.as<uint32_t>(), sc, s);
@@ -993,7 +985,7 @@ hipError_t TreeBuild::build(const float4* tri_sphere, const float4* tri_mt, cons
     M.T = T; M.ids = sids.as<uint32_t>(); M.box = bx; M.base = T;
     M.node = node.as<float4>(); M.size = size.as<uint32_t>();
     M.out = left.as<uint32_t>(); M.out_count = left_count.as<uint32_t>();
-    M.area = area.as<float>(); M.area_blocks = prim_blocks; M.cost = reinterpret_cast<float*>(cost.dev);
+    M.area = sums; M.area_blocks = prim_blocks; M.measure = measure;
     uint32_t groups = (T + MERGE_CHUNK - 1) / MERGE_CHUNK;
     M.last = groups == 1;
     k_tree_merge<true><<<groups, 1024, 0, s>>>(M);

@@ -2,7 +2,6 @@
 // surface, shading, hierarchy and traversal stages.
 #pragma once
 #include "fastdiv.hpp"
-#include "host_words.hpp"
 #include "rsh_internal.hpp"
 
 namespace rsh {
@@ -333,21 +332,23 @@ static_assert(sizeof(TreeNode) == 128, "a node is one cache line");
 
 constexpr uint32_t TREE_MAX_TRIANGLES = 1u << 29;      // places in a child word
 
+// What a build measures of the scene: the surface of the triangles' boxes over
+// that of the scene's, which is how many of them a line through the scene meets,
+// and half the latter.  Not finite where the surfaces are not.
+struct TreeMeasure {
+    float boxes, half_root;
+};
+
 struct TreeBuild {
     DevBuf nodes, records, bounds;                                          // what the traversal reads (parts of keep)
     // construction (parts of work)
-    DevBuf box, node, size, left, left_count, area, codes, ids, scodes, sids, queue, count;
+    DevBuf box, node, size, left, left_count, codes, ids, scodes, sids, queue, count;
     ScanScratch sc;                                                         // the sort's scratch (part of work)
     DevBuf keep, work;
-    HostWords cost;                                                         // float, as boxes() returns it
     hipError_t reserve(uint32_t T);
-    // Once a build has ended on its stream: the surface of the triangles' boxes
-    // over that of the scene's, which is how many of them a line through the
-    // scene meets (0 where it is not finite).
-    float boxes() const;
     // objects: per object (first triangle, ...), K of them tiling [0, T) in order
     hipError_t build(const float4* tri_sphere, const float4* tri_mt, const uint4* objects, uint32_t K, uint32_t T,
-                     hipStream_t s);
+                     TreeMeasure* measure, hipStream_t s);
     void release();
 };
 
@@ -370,7 +371,7 @@ struct TreeParams {
     const float4* obj_sphere;
     const uint4* obj_range;
     uint32_t algorithm, kind, hit_mode, line_only;
-    float boxes;                  // TreeBuild::boxes
+    float boxes;                  // TreeMeasure::boxes
     uint32_t frame;               // a frame's pass (0: a query's)
     uint32_t walk, small_stack;   // a test's (rsh_selfcheck_tree_walk)
     uint32_t stack;               // entries of a ray's stack to use (set by the launch)

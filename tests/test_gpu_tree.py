@@ -462,3 +462,58 @@ def test_small_captured_frames_are_no_slower_than_without_the_tree(engine, rsh, 
     tree = frame_ms(engine, cam, cfg, engine.GRAPH)
     walk(NO_TREE)
     assert tree < frame_ms(engine, cam, cfg, engine.GRAPH)
+
+
+def test_large_camera_passes_of_overlapping_scenes(engine, rsh, walk):
+    """Their camera pass takes the kernels that share candidates among
+    neighbours (mode 1 or 2), the others the tree (3): the same hits, eager and
+    replayed, and no slower than without the tree (measured at 0.85; with the
+    tree for every pass 1.3)."""
+    sc = rsh.scenes.soup_scene()
+    cfg = rsh.config.config0(1024, 1024).with_scene_bounds(sc)
+    cam = rsh.scenes.random_view(np.random.default_rng(1), 1024, 1024)
+    engine.load_scene(sc)
+    engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+    modes = list(engine.stats.pass_mode[:engine.stats.pass_count])
+    assert modes[0] in (1, 2) and set(modes[1:]) == {3}
+    got, px = [engine.pass_hits(i) for i in range(len(modes))], engine.pixels()
+    for _ in range(3):
+        engine.render(cam, cfg, flags=engine.GRAPH)
+        np.testing.assert_array_equal(engine.pixels(), px)
+    auto = [frame_ms(engine, cam, cfg, fl) for fl in (0, engine.GRAPH)]
+    walk(QUAD)
+    engine.render(cam, cfg, flags=engine.KEEP_PASSES)
+    assert list(engine.stats.pass_mode[:len(modes)]) == [3] * len(modes)
+    for i, g in enumerate(got):
+        np.testing.assert_array_equal(g, engine.pass_hits(i))
+    walk(NO_TREE)
+    for ms, fl in zip(auto, (0, engine.GRAPH)):
+        assert ms < frame_ms(engine, cam, cfg, fl)
+
+
+@pytest.mark.parametrize("scene", ["config0", "config1", "config2"])
+def test_camera_passes_of_other_scenes_keep_the_tree(engine, rsh, scene):
+    sc = getattr(rsh.scenes, scene + "_scene")()
+    cfg = rsh.config.config0(1920, 1080).with_scene_bounds(sc)
+    engine.load_scene(sc)
+    engine.render(getattr(rsh.scenes, scene + "_camera")(1920, 1080), cfg)
+    assert set(engine.stats.pass_mode[:engine.stats.pass_count]) == {3}
+
+
+def test_overlap_is_measured_again_after_an_update(engine, rsh):
+    """Objects pulled apart, and put back: the camera pass's kernels follow."""
+    sc = rsh.scenes.soup_scene()
+    cfg = rsh.config.config0(1024, 1024).with_scene_bounds(sc)
+    cam = rsh.scenes.random_view(np.random.default_rng(1), 1024, 1024)
+    engine.load_scene(sc)
+    K = sc.object_total
+    eye = np.tile(np.eye(4, dtype=np.float32), (K, 1, 1))
+    apart = eye.copy()
+    apart[:, :3, 3] = np.random.default_rng(2).uniform(-5e4, 5e4, (K, 3))
+    for m, tree in ((apart, True), (eye, False)):
+        engine.update_objects(m, eye, eye)
+        engine.render(cam, cfg)
+        assert (engine.stats.pass_mode[0] == 3) == tree
+        px = engine.pixels()
+        engine.render(cam, dataclasses.replace(cfg, traversal_prefilter=2))
+        np.testing.assert_array_equal(engine.pixels(), px)

@@ -362,6 +362,11 @@ rsh_status rsh_selfcheck_wait_deadline(uint32_t wait_ms, uint32_t block_ms, uint
  * to the rules of size.  small_stack: ray stacks of a few entries, so that most
  * rays take the path of a full one.  Results are the same in every mode. */
 rsh_status rsh_selfcheck_tree_walk(rsh_engine* e, uint32_t walk, uint32_t small_stack);
+/* The same for what a call does where device memory is short: the tree's
+ * construction buffers go back, at the next call the tree itself (the scene is
+ * then traced as one too large for it, until it is loaded again).
+ * RSH_INVALID_ARG where nothing is left to give back. */
+rsh_status rsh_selfcheck_give_back(rsh_engine* e);
 
 /* Device memory helpers (plain HIP calls, for callers without a HIP runtime
  * binding of their own). */

@@ -28,6 +28,7 @@
 
 #include "../../include/rsh.h"
 #include "rsh_kernels.hpp"
+#include "with_less.hpp"
 
 using namespace rsh;
 
@@ -81,6 +82,7 @@ struct Lane {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     std::string err;
+    bool no_memory = false;            // an allocation of the lane's failed
     size_t cap_slots = 0;
     DevBuf flags, keys, values, tvalues, bases, ckeys, cvalues, skeys, svalues;
     DevBuf rvalues, soff, rec0, rec1, nodes, aux, counters, dcounts;
@@ -126,6 +128,7 @@ struct rsh_engine {
     hipEvent_t frame_done = nullptr, copy_done = nullptr;
     bool copy_pending = false;
     std::string err;
+    bool no_memory = false;            // an allocation of the call's failed
 
     // scene
     uint32_t T = 0, K = 0, M = 0, L = 0;
@@ -223,6 +226,7 @@ bool fail(rsh_engine* e, const std::string& msg) {
         hipError_t _e = (call);                                                            \
         if (_e != hipSuccess) {                                                            \
             e->err = std::string(#call) + ": " + hipGetErrorString(_e);                    \
+            e->no_memory |= _e == hipErrorOutOfMemory;                                     \
             return RSH_HIP_ERROR;                                                          \
         }                                                                                  \
     } while (0)
@@ -234,6 +238,7 @@ bool fail(rsh_engine* e, const std::string& msg) {
         hipError_t _e = (call);                                                            \
         if (_e != hipSuccess) {                                                            \
             L.err = std::string(#call) + ": " + hipGetErrorString(_e);                     \
+            L.no_memory |= _e == hipErrorOutOfMemory;                                      \
             return RSH_HIP_ERROR;                                                          \
         }                                                                                  \
     } while (0)
@@ -253,6 +258,36 @@ bool fail(rsh_engine* e, const std::string& msg) {
             return RSH_HIP_ERROR;                                                          \
         }                                                                                  \
     } while (0)
+
+// What a tree holds goes back to a call that lacks memory: its construction
+// buffers (the next object update takes them again), then the tree (the scene is
+// then traced as one too large for it, until it is loaded again).
+bool give_back_tree(rsh_engine* e) {
+    if (!e->has_tree) return false;
+    for (Lane& l : e->lane)
+        if (l.stream) (void)hipStreamSynchronize(l.stream);
+    if (e->stream) (void)hipStreamSynchronize(e->stream);
+    (void)hipGetLastError();
+    if (e->tree.work.p) {
+        e->tree.work.release();
+    } else {
+        e->tree.release();
+        e->has_tree = false;
+    }
+    return true;
+}
+
+// A call on the engine, made again with less of the tree where memory is short.
+template <class Call>
+rsh_status within_memory(rsh_engine* e, Call call) {
+    return with_less(
+        [&] {
+            e->no_memory = e->lane[0].no_memory = e->lane[1].no_memory = false;
+            return call();
+        },
+        [&] { return e->no_memory || e->lane[0].no_memory || e->lane[1].no_memory; },
+        [&] { return give_back_tree(e); });
+}
 
 inline float4* f4p(const DevBuf& b) { return b.as<float4>(); }
 inline uint32_t* u32p(const DevBuf& b) { return b.as<uint32_t>(); }
@@ -528,6 +563,23 @@ double object_spread(const rsh_engine* e, const float* scale) {
         sum += r * r * ((double)h[5] - h[4] + 1.0);
     }
     return sum;
+}
+
+// The tree's buffers for the scene's T triangles.  A scene too large for the tree
+// (its 29-bit record places, or its memory) is traced by the kernels that test
+// every candidate.
+rsh_status reserve_tree(rsh_engine* e, uint32_t T) {
+    e->has_tree = T <= TREE_MAX_TRIANGLES;
+    if (!e->has_tree) return RSH_OK;
+    const hipError_t r = e->tree.reserve(T);
+    if (r != hipErrorOutOfMemory) {
+        HIP_OK(r);
+        return RSH_OK;
+    }
+    (void)hipGetLastError();
+    e->tree.release();
+    e->has_tree = false;
+    return RSH_OK;
 }
 
 // What chooses a pass's kernel, once the tree's build has ended.
@@ -1166,10 +1218,11 @@ rsh_status rsh_selfcheck_wait_deadline(uint32_t wait_ms, uint32_t block_ms, uint
     return st;
 }
 
-rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
-    if (!e || !s || !s->tri_pos || !s->tri_nrm || !s->tri_mat || !s->mat_diffuse || !s->mat_specular ||
+namespace {
+rsh_status load_scene(rsh_engine* e, const rsh_scene_desc* s) {
+    if (!s || !s->tri_pos || !s->tri_nrm || !s->tri_mat || !s->mat_diffuse || !s->mat_specular ||
         !s->object_spheres || !s->light_pos || !s->light_col || !s->light_int)
-        return e ? (fail(e, "load_scene: null argument"), RSH_INVALID_ARG) : RSH_INVALID_ARG;
+        return fail(e, "load_scene: null argument"), RSH_INVALID_ARG;
     if (s->triangle_total == 0 || s->object_total == 0 || s->light_total == 0 || s->material_total == 0) {
         e->err = "load_scene: empty scene";
         return RSH_INVALID_ARG;
@@ -1270,19 +1323,8 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     HIP_OK(hipMemcpyAsync(e->cl_base.p, base.data(), (size_t)K * 4, hipMemcpyHostToDevice, st));
     HIP_OK(hipMemcpyAsync(e->all_list.p, ident.data(), (size_t)K * 16, hipMemcpyHostToDevice, st));
     build_clusters(e, st);
-    // A scene too large for the tree (its 29-bit record places, or its memory)
-    // is traced by the kernels that test every candidate.
-    e->has_tree = T <= TREE_MAX_TRIANGLES;
-    if (e->has_tree) {
-        const hipError_t r = e->tree.reserve(T);
-        if (r == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            e->tree.release();
-            e->has_tree = false;
-        } else {
-            HIP_OK(r);
-        }
-    }
+    const rsh_status rs = reserve_tree(e, T);
+    if (rs != RSH_OK) return rs;
     if (e->has_tree)
         HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, e->measure_dev, st));
     HIP_OK(hipGetLastError());
@@ -1294,6 +1336,12 @@ rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
     e->ranges_tb = 0xFFFFFFFFu;
     e->scene_epoch++;
     return RSH_OK;
+}
+}  // namespace
+
+rsh_status rsh_engine_load_scene(rsh_engine* e, const rsh_scene_desc* s) {
+    if (!e) return RSH_INVALID_ARG;
+    return within_memory(e, [&] { return load_scene(e, s); });
 }
 
 }  // extern "C"
@@ -1806,38 +1854,11 @@ rsh_status render(rsh_engine* e, const ViewDesc* hv, uint32_t nv, const rsh_fram
     return RSH_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-rsh_status rsh_engine_render(rsh_engine* e, const rsh_camera* cam, const rsh_frame_config* cfgp, uint32_t fl,
-                             rsh_frame_stats* st) {
-    if (!e || !cam || !cfgp) return RSH_INVALID_ARG;
-    if (e->T == 0) { e->err = "render: no scene loaded"; return RSH_INVALID_ARG; }
-    const ViewDesc v = view_desc(*cam, 0, cfgp->width, cfgp->height);
-    return render(e, &v, 1, *cfgp, fl, st);
-}
-
-rsh_status rsh_engine_render_views(rsh_engine* e, const rsh_view* views, uint32_t n, const rsh_frame_config* cfgp,
-                                   uint32_t fl, rsh_frame_stats* st) {
-    if (!e || !views || !cfgp || n == 0) return RSH_INVALID_ARG;
-    if (e->T == 0) { e->err = "render_views: no scene loaded"; return RSH_INVALID_ARG; }
-    std::vector<ViewDesc> hv(n);
-    uint64_t off = 0;
-    for (uint32_t i = 0; i < n; i++) {
-        if (views[i].width == 0 || views[i].height == 0) { e->err = "render_views: empty view"; return RSH_INVALID_ARG; }
-        if (off > 0xFFFFFFFFull) { e->err = "render_views: batch exceeds 2^32 pixels"; return RSH_CAPACITY; }
-        hv[i] = view_desc(views[i].camera, (uint32_t)off, views[i].width, views[i].height);
-        off += (uint64_t)views[i].width * views[i].height;
-    }
-    if (off > 0xFFFFFFFFull) { e->err = "render_views: batch exceeds 2^32 pixels"; return RSH_CAPACITY; }
-    return render(e, hv.data(), n, *cfgp, fl, st);
-}
-
-rsh_status rsh_engine_trace(rsh_engine* e, const float* rays, const float* tmax, const uint32_t* segments, uint32_t n,
-                            uint32_t kind, const rsh_frame_config* cfgp, void* out, uint32_t fl, rsh_frame_stats* st) {
-    if (!e || !rays || !cfgp || !out || n == 0 || kind > 1 || (kind == 1 && !tmax)) {
-        if (e) e->err = "trace: null buffer, empty query, kind > 1 or any-hit without tmax";
+// rsh_engine_trace
+rsh_status trace(rsh_engine* e, const float* rays, const float* tmax, const uint32_t* segments, uint32_t n,
+                 uint32_t kind, const rsh_frame_config* cfgp, void* out, uint32_t fl, rsh_frame_stats* st) {
+    if (!rays || !cfgp || !out || n == 0 || kind > 1 || (kind == 1 && !tmax)) {
+        e->err = "trace: null buffer, empty query, kind > 1 or any-hit without tmax";
         return RSH_INVALID_ARG;
     }
     if (fl & 9u) { e->err = "trace: flags take counters (bit 1) and timing (bit 2) only"; return RSH_INVALID_ARG; }
@@ -1912,6 +1933,39 @@ rsh_status rsh_engine_trace(rsh_engine* e, const float* rays, const float* tmax,
     return RSH_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+rsh_status rsh_engine_render(rsh_engine* e, const rsh_camera* cam, const rsh_frame_config* cfgp, uint32_t fl,
+                             rsh_frame_stats* st) {
+    if (!e || !cam || !cfgp) return RSH_INVALID_ARG;
+    if (e->T == 0) { e->err = "render: no scene loaded"; return RSH_INVALID_ARG; }
+    const ViewDesc v = view_desc(*cam, 0, cfgp->width, cfgp->height);
+    return within_memory(e, [&] { return render(e, &v, 1, *cfgp, fl, st); });
+}
+
+rsh_status rsh_engine_render_views(rsh_engine* e, const rsh_view* views, uint32_t n, const rsh_frame_config* cfgp,
+                                   uint32_t fl, rsh_frame_stats* st) {
+    if (!e || !views || !cfgp || n == 0) return RSH_INVALID_ARG;
+    if (e->T == 0) { e->err = "render_views: no scene loaded"; return RSH_INVALID_ARG; }
+    std::vector<ViewDesc> hv(n);
+    uint64_t off = 0;
+    for (uint32_t i = 0; i < n; i++) {
+        if (views[i].width == 0 || views[i].height == 0) { e->err = "render_views: empty view"; return RSH_INVALID_ARG; }
+        if (off > 0xFFFFFFFFull) { e->err = "render_views: batch exceeds 2^32 pixels"; return RSH_CAPACITY; }
+        hv[i] = view_desc(views[i].camera, (uint32_t)off, views[i].width, views[i].height);
+        off += (uint64_t)views[i].width * views[i].height;
+    }
+    if (off > 0xFFFFFFFFull) { e->err = "render_views: batch exceeds 2^32 pixels"; return RSH_CAPACITY; }
+    return within_memory(e, [&] { return render(e, hv.data(), n, *cfgp, fl, st); });
+}
+
+rsh_status rsh_engine_trace(rsh_engine* e, const float* rays, const float* tmax, const uint32_t* segments, uint32_t n,
+                            uint32_t kind, const rsh_frame_config* cfgp, void* out, uint32_t fl, rsh_frame_stats* st) {
+    if (!e) return RSH_INVALID_ARG;
+    return within_memory(e, [&] { return trace(e, rays, tmax, segments, n, kind, cfgp, out, fl, st); });
+}
 rsh_status rsh_selfcheck_tree_walk(rsh_engine* e, uint32_t walk, uint32_t small_stack) {
     if (!e || walk > WALK_NONE) return RSH_INVALID_ARG;
     e->tree_walk = walk;
@@ -2050,9 +2104,9 @@ int rsh_device_count(void) {
 // frame by main.cpp:1131-1196, on the engine's scene: positions and normals
 // from the scene as loaded, then the per-triangle, cluster and sub-cluster
 // data rebuilt; captured frame graphs are dropped.
-rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const float* normal, const float* scale) {
-    if (!e || !model || !normal || !scale) return e ? (fail(e, "update_objects: null argument"), RSH_INVALID_ARG)
-                                                    : RSH_INVALID_ARG;
+namespace {
+rsh_status update_objects(rsh_engine* e, const float* model, const float* normal, const float* scale) {
+    if (!model || !normal || !scale) return fail(e, "update_objects: null argument"), RSH_INVALID_ARG;
     if (e->T == 0) { e->err = "update_objects: no scene loaded"; return RSH_INVALID_ARG; }
     HIP_OK(hipSetDevice(e->device));
     hipStream_t st = e->stream;
@@ -2090,6 +2144,10 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
     HIP_OK(hipMemcpy2DAsync(e->obj_sphere.p, 16, e->sph_tmp.p, 24, 16, K, hipMemcpyDeviceToDevice, st));
     launch_triangle_prep(f4p(e->tri_pos), T, f4p(e->tri_sphere), f4p(e->tri_mt), st);
     build_clusters(e, st);
+    if (e->has_tree) {          // its construction buffers may have been given back
+        const rsh_status rs = reserve_tree(e, T);
+        if (rs != RSH_OK) return rs;
+    }
     if (e->has_tree)
         HIP_OK(e->tree.build(f4p(e->tri_sphere), f4p(e->tri_mt), e->all_list.as<uint4>(), K, T, e->measure_dev, st));
     HIP_OK(hipGetLastError());
@@ -2099,6 +2157,16 @@ rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const fl
     drop_graph(e);
     e->scene_epoch++;
     return RSH_OK;
+}
+}  // namespace
+
+rsh_status rsh_engine_update_objects(rsh_engine* e, const float* model, const float* normal, const float* scale) {
+    if (!e) return RSH_INVALID_ARG;
+    return within_memory(e, [&] { return update_objects(e, model, normal, scale); });
+}
+
+rsh_status rsh_selfcheck_give_back(rsh_engine* e) {
+    return e && give_back_tree(e) ? RSH_OK : RSH_INVALID_ARG;
 }
 
 }  // extern "C"

@@ -133,7 +133,8 @@ NATIVE_SYMBOLS = ["rsh_engine_create", "rsh_engine_destroy", "rsh_last_error", "
                   "rsh_compat_configure", "rsh_compat_set_stream", "rsh_compat_set_exit_on_error",
                   "rsh_compat_status", "rsh_compat_error", "rsh_compat_reset_status", "rsh_selfcheck_rcp",
                   "rsh_object_spheres", "rsh_engine_update_objects", "rsh_engine_set_wait_timeout",
-                  "rsh_selfcheck_wait_deadline", "rsh_selfcheck_tree_walk", "rsh_engine_read_pass_order"]
+                  "rsh_selfcheck_wait_deadline", "rsh_selfcheck_tree_walk", "rsh_selfcheck_give_back",
+                  "rsh_engine_read_pass_order"]
 
 _lib = None
 
@@ -202,6 +203,8 @@ def lib():
     L.rsh_engine_set_wait_timeout.argtypes = [PV, u32]
     L.rsh_selfcheck_tree_walk.restype = C.c_int
     L.rsh_selfcheck_tree_walk.argtypes = [PV, u32, u32]
+    L.rsh_selfcheck_give_back.restype = C.c_int
+    L.rsh_selfcheck_give_back.argtypes = [PV]
     L.rsh_selfcheck_wait_deadline.restype = C.c_int
     L.rsh_selfcheck_wait_deadline.argtypes = [u32, u32, C.POINTER(u32)]
     for name, args in COMPAT_SIGNATURES.items():

@@ -517,3 +517,57 @@ def test_overlap_is_measured_again_after_an_update(engine, rsh):
         px = engine.pixels()
         engine.render(cam, dataclasses.replace(cfg, traversal_prefilter=2))
         np.testing.assert_array_equal(engine.pixels(), px)
+
+
+def test_tree_given_back_for_memory(rsh):
+    """Frames, queries, replays and object updates on an engine that has given
+    back the tree's construction buffers, and then the tree: the same results,
+    and the next load builds it again."""
+    sc = rsh.scenes.config1_scene(boxes=120)
+    cam = rsh.scenes.config1_camera(97, 61)
+    cfg = rsh.config.config1(97, 61).with_scene_bounds(sc)
+    K = sc.object_total
+    rng = np.random.default_rng(8)
+    eye = np.tile(np.eye(4, dtype=np.float32), (K, 1, 1))
+    moves = []
+    for _ in range(3):
+        m = eye.copy()
+        m[1:, :3, 3] = rng.uniform(-20.0, 20.0, (K - 1, 3))
+        moves.append(m)
+    rays = rays_at(rng, sc, 501)
+    steps = [None, moves[0], None, moves[1], moves[2]]
+
+    def results(e, m):
+        if m is not None:
+            e.update_objects(m, eye, eye)
+        e.render(cam, cfg)
+        out = [e.pixels()]
+        mode = e.stats.pass_mode[0]
+        for _ in range(2):
+            e.render(cam, cfg, flags=e.GRAPH)
+            out.append(e.pixels())
+        return out + [e.trace(rays, 0, cfg)], mode
+
+    e, ref = rsh.Engine(0), rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        ref.load_scene(sc)
+        # the construction buffers after the first step (an update takes them
+        # again), both parts after the second
+        for i, m in enumerate(steps):
+            got, mode = results(e, m)
+            want, _ = results(ref, m)
+            for g, w in zip(got, want):
+                np.testing.assert_array_equal(g, w)
+            assert (mode == 3) == (i < 2), (i, mode)
+            if i == 0:
+                assert e.L.rsh_selfcheck_give_back(e.h) == 0
+            elif i == 1:
+                assert e.L.rsh_selfcheck_give_back(e.h) == 0
+                assert e.L.rsh_selfcheck_give_back(e.h) == 0
+                assert e.L.rsh_selfcheck_give_back(e.h) != 0
+        e.load_scene(sc)
+        assert results(e, None)[1] == 3
+    finally:
+        e.close()
+        ref.close()

@@ -1551,11 +1551,13 @@ void launch_gather(const float* rays, const uint32_t* sorted_values, uint32_t N,
     if (N) k_gather<<<grid_for(N, 256, 65536), 256, 0, s>>>(g, N, ps, rec0, rec1);
 }
 
-// Up to 2^20 rays; beyond, a launch a level fills the chip with whole waves of
-// nodes and leaves the other lane's traversal its LDS (soft shadows, 3.9M rays:
-// 3.124 ms a frame so, 3.143 in one launch).
+// Up to 2^21 rays the one launch is the faster (queries, a launch a level and one:
+// 1.2M camera rays of the atrium 728 and 704 us, 2.1M 938 and 912, 2.1M shadow
+// rays 1142 and 1120; frames and batches of 1.3M to 3.7M pixels even).  Beyond, a
+// launch a level fills the chip with whole waves of nodes: 3M rays 1266 and 1269,
+// and soft shadows with 3.9M 3.124 ms a frame, 3.143 in one.
 bool fuses_levels(uint32_t N, uint32_t leaf, uint32_t branch, uint32_t depth) {
-    return N <= (1u << 20) && depth == 2 && leaf <= LEVELS_BLOCK && branch <= LEVELS_BLOCK && LEVELS_BLOCK % (leaf * branch) == 0;
+    return N <= (1u << 21) && depth == 2 && leaf <= LEVELS_BLOCK && branch <= LEVELS_BLOCK && LEVELS_BLOCK % (leaf * branch) == 0;
 }
 
 void launch_levels(const float* rays, const uint32_t* sorted_values, uint32_t N, const PassSizes* ps,

@@ -41,9 +41,10 @@ inline size_t sort_hist_bytes(uint64_t n) {
 // the expansion (34 us of a 100k-ray pass, whatever its size) but moves N pairs
 // a digit pass instead of C.  Up to 2^20 rays that costs less than it saves at
 // any N / C (100k shadow rays 270 -> 220 us; 1080p frame 2.88 -> 2.62 ms); above
-// it, 16 views in one pass of 1.9M rays and N / C = 5 take 8.1 ms sorted as rays
-// and 7.9 as packets, while with N / C < 2 the rays are again the cheaper (1M
-// incoherent rays 802 -> 755 us).
+// it, six 512x512 views in one pass of 1.6M rays take 2530 us sorted as rays and
+// 2490 as packets, 16 views with 1.9M and N / C = 5 8.1 ms and 7.9, while with
+// N / C < 2 the rays are again the cheaper (1M incoherent rays 802 -> 755 us; such
+// queries of 1.2M to 3M take the rays by this second condition).
 enum PackOrder : uint32_t { PACK_CHUNKS = 0, PACK_RAYS = 1, PACK_EITHER = 2 };
 __host__ __device__ inline bool sorts_rays(uint32_t N, uint32_t C) { return N <= (1u << 20) || N / 2 <= C; }
 

@@ -142,3 +142,25 @@ def test_small_frames(rsh, w, h):
         np.testing.assert_array_equal(pa, e.pixels())
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("w,h", [(2048, 1024), (2045, 1025), (2049, 1024), (1025, 1023)])
+def test_levels_of_large_passes(rsh, w, h):
+    """Camera passes about the 2^21 rays up to which both levels come from one
+    launch: the nodes of a hierarchy of three levels, made with a launch each,
+    start with the same two."""
+    sc = rsh.scenes.config0_scene()
+    cam = rsh.scenes.config0_camera(w, h)
+    e = rsh.Engine(0)
+    try:
+        e.load_scene(sc)
+        nodes = []
+        for depth in (2, 3):
+            cfg = dataclasses.replace(rsh.config.config0(w, h), depth=depth, bounces=0).with_scene_bounds(sc)
+            e.render(cam, cfg, flags=e.KEEP_ORDER)
+            nodes.append(e.pass_order(0)["nodes"].view(np.uint32))
+        n0 = -(-w * h // 8)
+        assert len(nodes[0]) == 2 * (n0 + -(-n0 // 8)) < len(nodes[1])
+        np.testing.assert_array_equal(nodes[0], nodes[1][:len(nodes[0])])
+    finally:
+        e.close()

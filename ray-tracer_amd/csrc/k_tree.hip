@@ -12,7 +12,7 @@
 // The tree is a four-wide bounding-box tree: a binary tree merged bottom up
 // over the triangles in Morton order, from which each wide node takes the
 // children of the largest surface.  It is rebuilt on the device at scene load
-// and after object updates (262,604 triangles: 0.41 ms, bound by the
+// and after object updates (262,604 triangles: 0.35 ms, bound by the
 // latency of its 26 launches and of the merging rounds).
 #include <algorithm>
 #include <cmath>
@@ -513,10 +513,10 @@ __global__ void __launch_bounds__(256) k_tree_records(EmitArgs A, const uint32_t
 // Four lanes per sorted ray (a quad): lane q tests child q of a node or
 // triangle q of a leaf; 16 rays, one wave, per workgroup.  Nearest child first;
 // the others wait on the ray's stack in LDS.
-// Large passes are bound by VALU issue (1080p atrium camera pass: 303M
-// instructions, 0.49 ms of issue in 0.52 ms) and the loads behind it, small
+// Large passes are bound by VALU issue (1080p atrium camera pass: 295M
+// instructions, 0.48 ms of issue in 0.52 ms) and the loads behind it, small
 // ones by the latency of the longest ray's steps (14k rays: 0.12 ms).  Waves
-// hide that latency: 8 a SIMD (64 VGPRs, 9 of the closest-hit kernel's spilled;
+// hide that latency: 8 a SIMD (64 VGPRs, 11 of the closest-hit kernel's spilled;
 // 3.0 / 4.5 KB of LDS) against 7 with 6 KB: 1080p atrium frame 2.97 -> 2.92 ms,
 // 16-view batch 8.65 -> 8.08, 1M diffuse rays 0.863 -> 0.806, soft shadows 3.45 ->
 // 3.15; 6 waves 2 to 4 % slower than 7, 5 waves 6 to 10 %.  One thread per ray needs half the
